@@ -14,16 +14,15 @@
 //     starts from init and its lookback stops at its own first tile.
 //     Segments of at most one wave chunk are scanned one per wave by a
 //     second kernel on the same stream (no descriptors, same bits);
-//   * sort_pairs: one block per segment of up to 8192 keys sorts it in LDS
-//     (LSD passes with the onesweep kernel's stable wave ranking); the
-//     longer segments of 4-byte keys (and 4-byte or no values) are sorted
+//   * sort_pairs: one block (or wave) per segment of up to 8192 keys sorts
+//     it in LDS (local_sort.hip); the longer segments of 4-byte keys (and 4-byte or no values) are sorted
 //     together by the segmented onesweep (one histogram launch, one launch
 //     per digit pass over all their tiles); 8-byte keys or values take one
 //     onesweep sort per longer segment.
 #include <algorithm>
 #include <vector>
 
-#include "radix.hpp"
+#include "local_sort.hpp"
 #include "reduce_tree.hpp"
 #include "segments.hpp"
 #include "workspace.hpp"
@@ -151,222 +150,85 @@ int seg_reduce_typed(raja_cdna4_segments_s* p, int op, const void* x, const void
   }
 }
 
-// ---- segmented sort: one block per short segment, LSD passes in LDS ----------------
+// ---- segmented sort: short segments in one block or wave each -----------------------
 
-template<typename K, typename V, bool HAS_VALS>
-struct BlockSortShape
+// The plan's sort records, built and uploaded at its first sort.
+int get_sort_table(raja_cdna4_segments_s* p, const raja_cdna4_segments_s::SortTable** out)
 {
-  static constexpr bool wide = sizeof(K) > 4 || (HAS_VALS && sizeof(V) > 4);
-  static constexpr int BLOCK = 512;
-  static constexpr int ITEMS = wide ? 8 : 16;
-  static constexpr int TILE = BLOCK * ITEMS;
-};
-
-template<typename K, typename V, bool DESC, bool HAS_VALS>
-__global__ __launch_bounds__(512) void block_sort_kernel(const K* in_keys, const V* in_vals,
-                                                         K* out_keys, V* out_vals,
-                                                         const rs::SortSeg* __restrict__ segs)
-{
-  using S = BlockSortShape<K, V, HAS_VALS>;
-  constexpr int BLOCK = S::BLOCK;
-  constexpr int ITEMS = S::ITEMS;
-  constexpr int NW = BLOCK / wave_size;
-  constexpr int WCHUNK = wave_size * ITEMS;
-  constexpr int P = (int)sizeof(K);
-  __shared__ K s_keys[S::TILE];
-  __shared__ V s_vals[HAS_VALS ? S::TILE : 1];
-  __shared__ uint32_t s_whist[NW * kRadix];
-  __shared__ uint32_t s_tstart[kRadix];
-  __shared__ uint32_t s_scan[kRadix / wave_size];
-
-  const int tid = threadIdx.x;
-  const int lane = lane_id();
-  const int wave = wave_id();
-  const rs::SortSeg sg = segs[blockIdx.x];
-  const int n = (int)sg.n;
-  K k[ITEMS];
-  V v[HAS_VALS ? ITEMS : 1];
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j)
+  std::lock_guard<std::mutex> g(p->lock);
+  raja_cdna4_segments_s::SortTable& t = p->sorts;
+  *out = &t;
+  if (t.built) return RAJA_CDNA4_SUCCESS;
+  std::vector<rs::SortSeg> small;
+  std::vector<rs::SortTile> recs;
+  const int64_t tile = rsort::seg_tile();
+  t.longer.clear();
+  for (int64_t g = 0; g < p->nseg; ++g)
   {
-    const int i = wave * WCHUNK + j * wave_size + lane;
-    k[j] = (i < n) ? in_keys[sg.in_keys + i] : K(0);
-    if (HAS_VALS) v[j] = (i < n) ? in_vals[sg.in_vals + i] : V(0);
+    const int64_t b = p->offsets[(size_t)g];
+    const int64_t len = p->offsets[(size_t)g + 1] - b;
+    if (len <= 1) continue;
+    if (len <= rsort::local_sort_max())
+    {
+      small.push_back(rs::SortSeg{b, b, b, b, len});
+      continue;
+    }
+    for (int64_t j = 0; j * tile < len; ++j)
+    {
+      recs.push_back(rs::SortTile{b, b, b, b, b, b, len, (uint32_t)j, (uint32_t)t.longer.size()});
+    }
+    t.longer.push_back(g);
   }
-  const uint64_t lt_mask = lanemask_lt();
-  for (int p = 0; p < P; ++p)
+  rsort::order_by_class(small, t.first);
+  t.ntiles = (int64_t)recs.size();
+  if (!small.empty() && !t.d_segs)
   {
-    const int shift = 8 * p;
-    for (int i = tid; i < NW * kRadix; i += BLOCK) s_whist[i] = 0u;
-    __syncthreads();
-    uint32_t rank[ITEMS];
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-    {
-      const int i = wave * WCHUNK + j * wave_size + lane;
-      const bool valid = i < n;
-      const uint32_t d = digit_of<K, DESC>(k[j], shift);
-      uint64_t peers = ballot(valid);
-#pragma unroll
-      for (int b = 0; b < 8; ++b)
-      {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t bal = ballot(bit);
-        peers &= bit ? bal : ~bal;
-      }
-      const uint32_t lower = (uint32_t)__popcll(peers & lt_mask);
-      uint32_t cnt = 0;
-      if (valid) cnt = s_whist[wave * kRadix + d];
-      rank[j] = cnt + lower;
-      if (valid && lower == 0) s_whist[wave * kRadix + d] = cnt + (uint32_t)__popcll(peers);
-    }
-    __syncthreads();
-    uint32_t ex_t = 0;
-    if (tid < kRadix)
-    {
-      uint32_t total = 0;
-#pragma unroll
-      for (int w = 0; w < NW; ++w)
-      {
-        const uint32_t c = s_whist[w * kRadix + tid];
-        s_whist[w * kRadix + tid] = total;
-        total += c;
-      }
-      uint32_t tot;
-      (void)wave_scan(total, rk::OpPlus<uint32_t>{}, 0u, ex_t, tot);
-      if (lane == 0) s_scan[wave] = tot;
-    }
-    __syncthreads();
-    if (tid < kRadix)
-    {
-      uint32_t ts = ex_t;
-      for (int w = 0; w < wave; ++w) ts += s_scan[w];
-      s_tstart[tid] = ts;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-    {
-      const int i = wave * WCHUNK + j * wave_size + lane;
-      if (i < n)
-      {
-        const uint32_t d = digit_of<K, DESC>(k[j], shift);
-        const uint32_t pos = s_tstart[d] + s_whist[wave * kRadix + d] + rank[j];
-        s_keys[pos] = k[j];
-        if (HAS_VALS) s_vals[pos] = v[j];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-    {
-      const int i = wave * WCHUNK + j * wave_size + lane;
-      if (i < n)
-      {
-        k[j] = s_keys[i];
-        if (HAS_VALS) v[j] = s_vals[i];
-      }
-    }
-    __syncthreads();
+    RC_HIP(hipMalloc(&t.d_segs, sizeof(rs::SortSeg) * small.size()));
+    RC_HIP(hipMemcpy(t.d_segs, small.data(), sizeof(rs::SortSeg) * small.size(), hipMemcpyHostToDevice));
   }
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j)
+  if (!recs.empty() && !t.d_tiles)
   {
-    const int i = wave * WCHUNK + j * wave_size + lane;
-    if (i < n)
-    {
-      out_keys[sg.out_keys + i] = k[j];
-      if (HAS_VALS) out_vals[sg.out_vals + i] = v[j];
-    }
+    RC_HIP(hipMalloc(&t.d_tiles, sizeof(rs::SortTile) * recs.size()));
+    RC_HIP(hipMemcpy(t.d_tiles, recs.data(), sizeof(rs::SortTile) * recs.size(), hipMemcpyHostToDevice));
   }
+  t.built = true;
+  return RAJA_CDNA4_SUCCESS;
 }
 
 template<typename K, typename V, bool HAS_VALS, bool DESC>
 int seg_sort(raja_cdna4_segments_s* p, K* keys, V* vals, int key_dtype, int val_bytes,
              hipStream_t s)
 {
-  using S = BlockSortShape<K, V, HAS_VALS>;
-  std::vector<rs::SortSeg> small;
-  std::vector<int64_t> big;
-  for (int64_t g = 0; g < p->nseg; ++g)
+  const raja_cdna4_segments_s::SortTable* tab = nullptr;
+  RC_TRY(get_sort_table(p, &tab));
+  if (tab->first[rsort::kLocalClasses] > 0)
   {
-    const int64_t b = p->offsets[(size_t)g];
-    const int64_t len = p->offsets[(size_t)g + 1] - b;
-    if (len <= 1) continue;
-    if (len <= S::TILE) small.push_back(rs::SortSeg{b, b, b, b, len});
-    else big.push_back(g);
-  }
-  if (!small.empty())
-  {
-    rc::StreamCtx* c = nullptr;
-    RC_TRY(rc::get_ctx(s, &c));
-    // short-segment records: uploaded once per plan and block shape
-    rs::SortSeg* d_segs = nullptr;
-    {
-      std::lock_guard<std::mutex> g(p->lock);
-      auto it = p->sort_segs.find((int64_t)S::TILE);
-      if (it == p->sort_segs.end())
-      {
-        RC_HIP(hipMalloc(&d_segs, sizeof(rs::SortSeg) * small.size()));
-        RC_HIP(hipMemcpy(d_segs, small.data(), sizeof(rs::SortSeg) * small.size(), hipMemcpyHostToDevice));
-        it = p->sort_segs.emplace((int64_t)S::TILE, d_segs).first;
-      }
-      d_segs = it->second;
-    }
     rc::TimedScope ts("segmented_block_sort", s);
-    hipLaunchKernelGGL((block_sort_kernel<K, V, DESC, HAS_VALS>), dim3((unsigned)small.size()),
-                       dim3(S::BLOCK), 0, s, keys, vals, keys, vals, (const rs::SortSeg*)d_segs);
-    RC_HIP(hipGetLastError());
+    RC_TRY(rsort::local_sort_batch(key_dtype, HAS_VALS ? val_bytes : 0, DESC ? 1 : 0, keys, vals, keys,
+                                   vals, tab->d_segs, tab->first, s));
   }
-  if (big.empty()) return RAJA_CDNA4_SUCCESS;
+  if (tab->longer.empty()) return RAJA_CDNA4_SUCCESS;
   if constexpr (sizeof(K) == 4 && (!HAS_VALS || sizeof(V) == 4))
   {
-    // Every longer segment in one segmented onesweep: tile records built
-    // once per plan; alternates, histograms and descriptors from the
-    // stream's scratch.
-    const int64_t tile = rsort::seg_tile();
-    raja_cdna4_segments_s::SortTable tab;
-    {
-      std::lock_guard<std::mutex> g(p->lock);
-      auto it = p->sort_tables.find((int64_t)S::TILE);
-      if (it == p->sort_tables.end())
-      {
-        std::vector<rs::SortTile> recs;
-        for (size_t r = 0; r < big.size(); ++r)
-        {
-          const int64_t b = p->offsets[(size_t)big[r]];
-          const int64_t len = p->offsets[(size_t)big[r] + 1] - b;
-          for (int64_t j = 0; j * tile < len; ++j)
-          {
-            recs.push_back(rs::SortTile{b, b, b, b, b, b, len, (uint32_t)j, (uint32_t)r});
-          }
-        }
-        raja_cdna4_segments_s::SortTable t;
-        t.ntiles = (int64_t)recs.size();
-        t.nranges = (int64_t)big.size();
-        RC_HIP(hipMalloc(&t.d_tiles, sizeof(rs::SortTile) * recs.size()));
-        RC_HIP(hipMemcpy(t.d_tiles, recs.data(), sizeof(rs::SortTile) * recs.size(),
-                         hipMemcpyHostToDevice));
-        it = p->sort_tables.emplace((int64_t)S::TILE, t).first;
-      }
-      tab = it->second;
-    }
+    // Every longer segment in one segmented onesweep: alternates, histograms
+    // and descriptors from the stream's scratch.
+    const int64_t nranges = (int64_t)tab->longer.size();
     rc::StreamCtx* c = nullptr;
     RC_TRY(rc::get_ctx(s, &c));
     const size_t kb = rc::align_up((size_t)p->total * sizeof(K), 256);
     const size_t vb = HAS_VALS ? rc::align_up((size_t)p->total * sizeof(V), 256) : 0;
-    RC_TRY(rc::ensure_tmp(c, kb + vb + rsort::seg_hist_bytes(tab.nranges)));
-    RC_TRY(rc::ensure_sort_desc(c, rsort::seg_desc_bytes(tab.ntiles)));
+    RC_TRY(rc::ensure_tmp(c, kb + vb + rsort::seg_hist_bytes(nranges)));
+    RC_TRY(rc::ensure_sort_desc(c, rsort::seg_desc_bytes(tab->ntiles)));
     char* tmp = (char*)c->tmp;
     return rsort::seg_sort_table(key_dtype, HAS_VALS ? 4 : 0, DESC ? 1 : 0, keys, vals, keys, vals,
-                                 tmp, HAS_VALS ? (void*)(tmp + kb) : nullptr, tab.d_tiles,
-                                 tab.ntiles, tab.nranges, (uint32_t*)(tmp + kb + vb),
+                                 tmp, HAS_VALS ? (void*)(tmp + kb) : nullptr, tab->d_tiles,
+                                 tab->ntiles, nranges, (uint32_t*)(tmp + kb + vb),
                                  (uint32_t*)c->sort_desc, s);
   }
   else
   {
     // 8-byte keys or values: one onesweep sort per longer segment.
-    for (int64_t g : big)
+    for (int64_t g : tab->longer)
     {
       const int64_t b = p->offsets[(size_t)g], len = p->offsets[(size_t)g + 1] - b;
       RC_TRY(raja_cdna4_sort_pairs(key_dtype, keys + b, HAS_VALS ? (void*)(vals + b) : nullptr,
@@ -427,16 +289,15 @@ int table_sum_f64(const double* base, const rs::TileRec* d_tiles, int64_t ntiles
   return RAJA_CDNA4_SUCCESS;
 }
 
-int64_t block_sort_max() { return BlockSortShape<uint32_t, uint32_t, true>::TILE; }
+int64_t block_sort_max() { return rsort::local_sort_max(); }
 
-int block_sort_u32_i32(const uint32_t* base, const rs::SortSeg* d_segs, int64_t nseg, hipStream_t s)
+int block_sort_u32_i32(const uint32_t* base, const rs::SortSeg* d_segs,
+                       const int64_t (&first)[rsort::kLocalClasses + 1], hipStream_t s)
 {
-  if (nseg == 0) return RAJA_CDNA4_SUCCESS;
+  if (first[rsort::kLocalClasses] == 0) return RAJA_CDNA4_SUCCESS;
   rc::TimedScope ts("segmented_block_sort", s);
-  hipLaunchKernelGGL((block_sort_kernel<uint32_t, uint32_t, false, true>), dim3((unsigned)nseg),
-                     dim3(512), 0, s, base, base, (uint32_t*)base, (uint32_t*)base, d_segs);
-  RC_HIP(hipGetLastError());
-  return RAJA_CDNA4_SUCCESS;
+  return rsort::local_sort_batch(RAJA_CDNA4_U32, 4, 0, base, base, (void*)base, (void*)base, d_segs,
+                                 first, s);
 }
 }  // namespace rws
 
@@ -484,8 +345,8 @@ int raja_cdna4_segments_destroy(raja_cdna4_segments_s* p)
     if (kv.second.d_count) RC_HIP(hipFree(kv.second.d_count));
     if (kv.second.d_short) RC_HIP(hipFree(kv.second.d_short));
   }
-  for (auto& kv : p->sort_segs) RC_HIP(hipFree(kv.second));
-  for (auto& kv : p->sort_tables) RC_HIP(hipFree(kv.second.d_tiles));
+  if (p->sorts.d_segs) RC_HIP(hipFree(p->sorts.d_segs));
+  if (p->sorts.d_tiles) RC_HIP(hipFree(p->sorts.d_tiles));
   if (p->d_offsets) RC_HIP(hipFree(p->d_offsets));
   delete p;
   return RAJA_CDNA4_SUCCESS;

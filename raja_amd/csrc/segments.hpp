@@ -84,16 +84,20 @@ struct raja_cdna4_segments_s
   std::vector<int64_t> offsets;  // nseg + 1, host copy
   int64_t* d_offsets = nullptr;
   std::map<std::pair<int64_t, int64_t>, rs::TileTable> tables;  // (tile, short limit)
-  std::map<int64_t, rs::SortSeg*> sort_segs;  // per block shape: short-segment records
-  // tile records of the segments longer than one block sort (segmented
-  // onesweep), per block-sort limit
+  // The segments as the batched sort takes them, built at the plan's first
+  // sort: records of those one block sorts, by length class (rsort::
+  // order_by_class), tile records of the longer ones (segmented onesweep) and
+  // the longer ones' indices.
   struct SortTable
   {
+    bool built = false;
+    rs::SortSeg* d_segs = nullptr;
+    int64_t first[5] = {0, 0, 0, 0, 0};
     rs::SortTile* d_tiles = nullptr;
     int64_t ntiles = 0;
-    int64_t nranges = 0;
+    std::vector<int64_t> longer;
   };
-  std::map<int64_t, SortTable> sort_tables;
+  SortTable sorts;
   std::mutex lock;
 };
 

@@ -186,6 +186,7 @@ struct BatchPlan
   std::vector<uint32_t> sum_first, sum_count;
   std::vector<int64_t> sum_out;
   std::vector<rs::SortSeg> sorts;       // one block each (block_sort_max() keys or fewer)
+  int64_t sort_first[rsort::kLocalClasses + 1] = {};  // first record of each length class
   std::vector<rs::SortTile> sort_tiles;  // tiles of the longer sorts (segmented onesweep)
   int64_t sort_ranges = 0, alt_elems = 0;
   uintptr_t sum_base = 0, scan_base = 0, sort_base = 0;
@@ -278,6 +279,7 @@ struct BatchPlan
         alt_elems += (r.n + 63) / 64 * 64;
       }
     }
+    rsort::order_by_class(sorts, sort_first);
     size_t o = 0;
     auto place = [&](size_t bytes) {
       const size_t at = o;
@@ -410,7 +412,7 @@ int launch_batch(raja_cdna4_server_s* sv, Slot& slot, char* dev, hipStream_t s)
     RC_HIP(hipEventRecord(slot.uploaded, sv->upload));
     RC_HIP(hipStreamWaitEvent(s, slot.uploaded, 0));
   }
-  // The block sorts (a few dozen blocks, about 35 us) run on the upload
+  // The block sorts (a few dozen blocks) run on the upload
   // stream, after the upload, beside the unit's other kernels; the unit's
   // stream waits for them at its end.
   const bool side = !p.sorts.empty() && (!p.sum_out.empty() || !p.scan_tiles.empty() ||
@@ -419,7 +421,7 @@ int launch_batch(raja_cdna4_server_s* sv, Slot& slot, char* dev, hipStream_t s)
   {
     hipStream_t bs = side ? sv->upload : s;
     RC_TRY(rws::block_sort_u32_i32((const uint32_t*)p.sort_base, (const rs::SortSeg*)(dev + p.o_sorts),
-                                   (int64_t)p.sorts.size(), bs));
+                                   p.sort_first, bs));
     if (side) RC_HIP(hipEventRecord(slot.sorted, bs));
   }
   if (!p.sum_out.empty())

@@ -23,6 +23,7 @@
 //      launch or device counter is needed.
 // Ranking follows input order inside a wave (item j, then lane) and across
 // waves and tiles, so the sort is stable.
+#include "local_sort.hpp"
 #include "ops.hpp"
 #include "radix.hpp"
 #include "runtime.hpp"
@@ -898,6 +899,14 @@ int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
   {
     return rc::set_error(RAJA_CDNA4_ERROR_UNSUPPORTED, "sort length %lld exceeds %lld",
                          (long long)n, (long long)kMaxSortN);
+  }
+  if (n <= rsort::local_sort_max())
+  {
+    // One launch of one block (local_sort.hip) instead of a clear, a
+    // histogram and a pass per digit over one tile.
+    rc::TimedScope ts("block_sort", s);
+    return rsort::local_sort_one(rk::dtype_code<K>(), HAS_VALS ? (int)sizeof(V) : 0, DESC ? 1 : 0, keys,
+                                 vals, keys, vals, n, s);
   }
   using S = SortShape<K, V, HAS_VALS>;
   if (items < 0)

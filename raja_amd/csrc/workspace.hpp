@@ -4,6 +4,7 @@
 // admission.  All are asynchronous on `s` and never synchronise it.
 #pragma once
 
+#include "local_sort.hpp"
 #include "segments.hpp"
 
 namespace rws
@@ -43,8 +44,9 @@ int64_t scan_tile_i32();
 int table_exclusive_i32(const int32_t* in_base, int32_t* out_base, const rs::TileRec* d_tiles,
                         int64_t ntiles, void* ws, hipStream_t s);
 
-// Stable sorts of nseg (uint32, int32) ranges of at most block_sort_max()
-// pairs, one block each.
+// Stable sorts of (uint32, int32) ranges of at most block_sort_max() pairs,
+// one block or wave each, by records ordered by rsort::order_by_class.
 int64_t block_sort_max();
-int block_sort_u32_i32(const uint32_t* base, const rs::SortSeg* d_segs, int64_t nseg, hipStream_t s);
+int block_sort_u32_i32(const uint32_t* base, const rs::SortSeg* d_segs,
+                       const int64_t (&first)[rsort::kLocalClasses + 1], hipStream_t s);
 }  // namespace rws
