@@ -6,10 +6,9 @@
 // rocPRIM's temp-storage query and allocation) each.  Here one plan holds
 // the device segment/tile table, and each batched call is one or two
 // kernels over all segments:
-//   * reduce: one block per tile of every segment, then one wave per
-//     segment folds its tile values -- the same tree as the span reduction
-//     (reduce_tree.hpp), so a segment's result is bit-identical alone and in
-//     the batch;
+//   * reduce: one block per quad and one wave per short segment, then one
+//     wave folds the quad values of each segment of several -- the same tree as the span reduction (reduce_tree.hpp), so a segment's
+//     result is bit-identical alone and in the batch;
 //   * scan: the single-pass scan kernel over the tile table; each segment
 //     starts from init and its lookback stops at its own first tile.
 //     Segments of at most one wave chunk are scanned one per wave by a
@@ -19,6 +18,8 @@
 //     together by the segmented onesweep (one histogram launch, one launch
 //     per digit pass over all their tiles); 8-byte keys or values take one
 //     onesweep sort per longer segment.
+#include <string.h>
+
 #include <algorithm>
 #include <vector>
 
@@ -43,28 +44,17 @@ int get_table(raja_cdna4_segments_s* p, int64_t tile, const TileTable** out, int
   TileTable t;
   t.tile = tile;
   std::vector<TileRec> recs, shorts;
-  std::vector<uint32_t> first((size_t)p->nseg), count((size_t)p->nseg);
   for (int64_t s = 0; s < p->nseg; ++s)
   {
     const int64_t b = p->offsets[(size_t)s], len = p->offsets[(size_t)s + 1] - b;
     if (len > 0 && len <= short_max)
-    {
       shorts.push_back(TileRec{b, len, 0u, (uint32_t)s, 0});
-      first[(size_t)s] = (uint32_t)recs.size();
-      count[(size_t)s] = 0;
-      continue;
-    }
-    const int64_t nt = rc::ceil_div(len, tile);
-    first[(size_t)s] = (uint32_t)recs.size();
-    count[(size_t)s] = (uint32_t)nt;
-    t.max_count = std::max(t.max_count, (uint32_t)nt);
-    for (int64_t j = 0; j < nt; ++j) recs.push_back(TileRec{b, len, (uint32_t)j, (uint32_t)s, 0});
+    else
+      append_tiles(recs, b, len, b, (uint32_t)s, tile);
   }
   t.ntiles = (int64_t)recs.size();
   t.nshort = (int64_t)shorts.size();
   RC_HIP(hipMalloc(&t.d_tiles, sizeof(TileRec) * (recs.size() + 1)));
-  RC_HIP(hipMalloc(&t.d_first, sizeof(uint32_t) * (first.size() + 1)));
-  RC_HIP(hipMalloc(&t.d_count, sizeof(uint32_t) * (count.size() + 1)));
   RC_HIP(hipMalloc(&t.d_short, sizeof(TileRec) * (shorts.size() + 1)));
   if (!recs.empty())
   {
@@ -73,11 +63,6 @@ int get_table(raja_cdna4_segments_s* p, int64_t tile, const TileTable** out, int
   if (!shorts.empty())
   {
     RC_HIP(hipMemcpy(t.d_short, shorts.data(), sizeof(TileRec) * shorts.size(), hipMemcpyHostToDevice));
-  }
-  if (!first.empty())
-  {
-    RC_HIP(hipMemcpy(t.d_first, first.data(), sizeof(uint32_t) * first.size(), hipMemcpyHostToDevice));
-    RC_HIP(hipMemcpy(t.d_count, count.data(), sizeof(uint32_t) * count.size(), hipMemcpyHostToDevice));
   }
   auto ins = p->tables.emplace(key, t);
   *out = &ins.first->second;
@@ -94,16 +79,110 @@ using namespace RAJA::cdna4::dev;
 
 constexpr int kSegMaxGroups = 64;  // segments of up to 4096 tiles
 
+// Blocks 0 .. nquads-1 compute one quad each (a segment of one quad is done
+// there, result and init included); the blocks after them do a short segment
+// (short_elems() or fewer) per wave, which fills the tail.
+template<typename T, typename Op>
+__global__ __launch_bounds__(rt::kBlock) void seg_quads_kernel(
+    const T* __restrict__ x, const rs::TileRec* __restrict__ quads, int64_t nquads,
+    const rs::TileRec* __restrict__ shorts, int64_t nshort,
+    typename Op::acc_t* __restrict__ partials, typename Op::acc_t init, rt::ResultOut<Op> out)
+{
+  using acc_t = typename Op::acc_t;
+  __shared__ acc_t s_w[rt::kBlockWaves];
+  if ((int64_t)blockIdx.x < nquads)
+  {
+    const rs::TileRec r = quads[blockIdx.x];
+    const acc_t v = rt::fold_quad<T, Op>(x + r.seg_start, r.seg_len, r.j, s_w);
+    if (threadIdx.x != 0) return;
+    if (r.seg_len > rt::quad_elems<T, Op>())
+    {
+      partials[blockIdx.x] = v;
+      return;
+    }
+    const acc_t id = Op::ident();
+    out.put(r.seg, Op::with_init(init, rt::fold4<Op>(v, id, id, id)));
+    return;
+  }
+  const int64_t q = ((int64_t)blockIdx.x - nquads) * rt::kBlockWaves +
+                    __builtin_amdgcn_readfirstlane(wave_id());
+  if (q >= nshort) return;
+  const rs::TileRec r = shorts[q];
+  const acc_t v = rt::fold_short<T, Op>(x + r.seg_start, r.seg_len);
+  if (lane_id() == 0) out.put(r.seg, Op::with_init(init, v));
+}
+
+// One tile per block (the server's batches: a quarter of the records to
+// build and upload, and enough tiles without the finer cut).
 template<typename T, typename Op>
 __global__ __launch_bounds__(rt::kBlock) void seg_tiles_kernel(
     const T* __restrict__ x, const rs::TileRec* __restrict__ tiles,
     typename Op::acc_t* __restrict__ partials)
 {
   using acc_t = typename Op::acc_t;
-  __shared__ acc_t s_scratch[max_waves];
+  __shared__ acc_t s_w[16];
   const rs::TileRec r = tiles[blockIdx.x];
-  const acc_t v = rt::fold_tile<T, Op>(x + r.seg_start, r.seg_len, r.j, s_scratch);
+  const acc_t v = rt::fold_tile<T, Op>(x + r.seg_start, r.seg_len, r.j, s_w);
   if (threadIdx.x == 0) partials[blockIdx.x] = v;
+}
+
+// The plan's reduction table for quads of `quad` elements and one wave for
+// segments of up to short_max, built and uploaded at its first use.
+int get_reduce_table(raja_cdna4_segments_s* p, int64_t quad, int64_t short_max, const rs::ReduceTable** out)
+{
+  std::lock_guard<std::mutex> g(p->lock);
+  auto it = p->reduce_tables.find(quad);
+  if (it != p->reduce_tables.end())
+  {
+    *out = &it->second;
+    return RAJA_CDNA4_SUCCESS;
+  }
+  rs::ReduceTable t;
+  std::vector<rs::TileRec> quads, shorts;
+  std::vector<uint32_t> first, count;
+  std::vector<int64_t> index;
+  for (int64_t s = 0; s < p->nseg; ++s)
+  {
+    const int64_t b = p->offsets[(size_t)s], len = p->offsets[(size_t)s + 1] - b;
+    if (len <= short_max)
+    {
+      shorts.push_back(rs::TileRec{b, len, 0u, (uint32_t)s, 0});
+      continue;
+    }
+    const int64_t nq = rc::ceil_div(len, quad);
+    if (nq > 1)
+    {
+      first.push_back((uint32_t)quads.size());
+      count.push_back((uint32_t)nq);
+      index.push_back(s);
+    }
+    t.max_count = std::max(t.max_count, (uint32_t)nq);
+    rs::append_tiles(quads, b, len, b, (uint32_t)s, quad);
+  }
+  t.nquads = (int64_t)quads.size();
+  t.nlong = (int64_t)first.size();
+  t.nshort = (int64_t)shorts.size();
+  // one allocation and one copy for the five arrays (8-byte ones first)
+  std::vector<char> image;
+  auto place = [&image](const auto& v) {
+    const size_t at = image.size();
+    const size_t bytes = sizeof(v[0]) * v.size();
+    image.resize(at + bytes);
+    if (bytes) ::memcpy(image.data() + at, v.data(), bytes);
+    return at;
+  };
+  image.reserve(sizeof(rs::TileRec) * (quads.size() + shorts.size()) + 16 * first.size() + 64);
+  const size_t at_quads = place(quads), at_shorts = place(shorts), at_out = place(index),
+               at_first = place(first), at_count = place(count);
+  RC_HIP(hipMalloc((void**)&t.mem, image.size() + 1));
+  if (!image.empty()) RC_HIP(hipMemcpy(t.mem, image.data(), image.size(), hipMemcpyHostToDevice));
+  t.d_quads = (const rs::TileRec*)(t.mem + at_quads);
+  t.d_short = (const rs::TileRec*)(t.mem + at_shorts);
+  t.d_out = (const int64_t*)(t.mem + at_out);
+  t.d_first = (const uint32_t*)(t.mem + at_first);
+  t.d_count = (const uint32_t*)(t.mem + at_count);
+  *out = &p->reduce_tables.emplace(quad, t).first->second;
+  return RAJA_CDNA4_SUCCESS;
 }
 
 template<typename T, typename Op>
@@ -111,28 +190,30 @@ int seg_reduce(raja_cdna4_segments_s* p, const T* x, typename Op::acc_t init,
                typename Op::acc_t* out, hipStream_t s)
 {
   using acc_t = typename Op::acc_t;
-  const rs::TileTable* tab = nullptr;
-  RC_TRY(rs::get_table(p, rt::tile_elems<T>(), &tab));
-  if (tab->max_count > (uint32_t)kSegMaxGroups * 64)
+  if (p->nseg == 0) return RAJA_CDNA4_SUCCESS;
+  const rs::ReduceTable* tab = nullptr;
+  RC_TRY(get_reduce_table(p, rt::quad_elems<T, Op>(), rt::short_elems<T, Op>(), &tab));
+  if (tab->max_count > (uint32_t)kSegMaxGroups * 64 * 4)
   {
     return rc::set_error(RAJA_CDNA4_ERROR_UNSUPPORTED, "segment too long for the batched reduce");
   }
-  if (p->nseg == 0) return RAJA_CDNA4_SUCCESS;
   rc::StreamCtx* c = nullptr;
   RC_TRY(rc::get_ctx(s, &c));
-  RC_TRY(rc::ensure_tmp(c, (size_t)(tab->ntiles + 1) * sizeof(acc_t)));
+  RC_TRY(rc::ensure_tmp(c, (size_t)(tab->nquads + 1) * sizeof(acc_t)));
   acc_t* partials = (acc_t*)c->tmp;
   rc::TimedScope ts("segmented_reduce", s);
-  if (tab->ntiles > 0)
+  const int64_t grid = tab->nquads + rc::ceil_div(tab->nshort, rt::kBlockWaves);
+  hipLaunchKernelGGL((seg_quads_kernel<T, Op>), dim3((unsigned)grid), dim3(rt::kBlock), 0, s, x,
+                     tab->d_quads, tab->nquads, tab->d_short,
+                     tab->nshort, partials, init, rt::ResultOut<Op>{out});
+  RC_HIP(hipGetLastError());
+  if (tab->nlong > 0)
   {
-    hipLaunchKernelGGL((seg_tiles_kernel<T, Op>), dim3((unsigned)tab->ntiles), dim3(rt::kBlock), 0, s,
-                       x, (const rs::TileRec*)tab->d_tiles, partials);
+    hipLaunchKernelGGL((rt::final_kernel<Op, 1, kSegMaxGroups, true>), dim3((unsigned)tab->nlong),
+                       dim3(64), 0, s, partials, tab->d_first, tab->d_count, (int64_t)0, init,
+                       rt::ResultOut<Op>{out}, tab->d_out);
     RC_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL((rt::final_kernel<Op, 1, kSegMaxGroups>), dim3((unsigned)p->nseg), dim3(64), 0, s,
-                     partials, (const uint32_t*)tab->d_first, (const uint32_t*)tab->d_count,
-                     (int64_t)0, init, out, (const int64_t*)nullptr);
-  RC_HIP(hipGetLastError());
   return RAJA_CDNA4_SUCCESS;
 }
 
@@ -264,9 +345,9 @@ int seg_sort_key(raja_cdna4_segments_s* p, int kd, void* keys, void* vals, int v
 
 namespace rws
 {
-int64_t sum_tile_f64() { return rt::tile_elems<double>(); }
+int64_t sum_tile_f64() { return rt::tile_elems<double, rk::OpPlus<double>>(); }
 
-int64_t sum_batch_max() { return (int64_t)kSegMaxGroups * 64 * rt::tile_elems<double>(); }
+int64_t sum_batch_max() { return (int64_t)kSegMaxGroups * 64 * rt::tile_elems<double, rk::OpPlus<double>>(); }
 
 int table_sum_f64(const double* base, const rs::TileRec* d_tiles, int64_t ntiles,
                   const uint32_t* d_first, const uint32_t* d_count, int64_t nseg,
@@ -282,9 +363,9 @@ int table_sum_f64(const double* base, const rs::TileRec* d_tiles, int64_t ntiles
                        base, d_tiles, partials);
     RC_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL((rt::final_kernel<Op, 1, kSegMaxGroups>), dim3((unsigned)nseg), dim3(64), 0, s,
-                     (const double*)partials, d_first, d_count, (int64_t)0, 0.0, (double*)base,
-                     d_out_index);
+  hipLaunchKernelGGL((rt::final_kernel<Op, 1, kSegMaxGroups, false>), dim3((unsigned)nseg), dim3(64), 0, s,
+                     (const double*)partials, d_first, d_count, (int64_t)0, 0.0,
+                     rt::ResultOut<Op>{(double*)base}, d_out_index);
   RC_HIP(hipGetLastError());
   return RAJA_CDNA4_SUCCESS;
 }
@@ -341,10 +422,9 @@ int raja_cdna4_segments_destroy(raja_cdna4_segments_s* p)
   for (auto& kv : p->tables)
   {
     if (kv.second.d_tiles) RC_HIP(hipFree(kv.second.d_tiles));
-    if (kv.second.d_first) RC_HIP(hipFree(kv.second.d_first));
-    if (kv.second.d_count) RC_HIP(hipFree(kv.second.d_count));
     if (kv.second.d_short) RC_HIP(hipFree(kv.second.d_short));
   }
+  for (auto& kv : p->reduce_tables) RC_HIP(hipFree(kv.second.mem));
   if (p->sorts.d_segs) RC_HIP(hipFree(p->sorts.d_segs));
   if (p->sorts.d_tiles) RC_HIP(hipFree(p->sorts.d_tiles));
   if (p->d_offsets) RC_HIP(hipFree(p->d_offsets));

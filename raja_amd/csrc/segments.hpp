@@ -58,20 +58,31 @@ inline void append_tiles(std::vector<TileRec>& recs, int64_t start, int64_t len,
   }
 }
 
-// Tiles of one tile size: tile records plus, per segment, its first tile
-// and tile count.  A table built with a short-segment limit holds the tiles
-// of the longer segments only, and the short ones (1 .. limit elements) as
-// a separate list of one record each.
+// Tile records of one tile size.  A table built with a short-segment limit
+// holds the tiles of the longer segments only, and the short ones (1 .. limit
+// elements) as a separate list of one record each.
 struct TileTable
 {
   int64_t tile = 0;
   int64_t ntiles = 0;
   TileRec* d_tiles = nullptr;
-  uint32_t* d_first = nullptr;
-  uint32_t* d_count = nullptr;
-  uint32_t max_count = 0;
   int64_t nshort = 0;
   TileRec* d_short = nullptr;
+};
+
+// A plan's segments as the batched reduction takes them, per quad size: one
+// record for each short one (empty ones too), quad records of the others, and
+// the first quad, quad count and output index of those of several quads.
+struct ReduceTable
+{
+  int64_t nquads = 0, nlong = 0, nshort = 0;
+  uint32_t max_count = 0;  // quads of the longest segment
+  char* mem = nullptr;  // one allocation holds the arrays
+  const TileRec* d_quads = nullptr;
+  const TileRec* d_short = nullptr;
+  const uint32_t* d_first = nullptr;
+  const uint32_t* d_count = nullptr;
+  const int64_t* d_out = nullptr;
 };
 
 }  // namespace rs
@@ -83,7 +94,8 @@ struct raja_cdna4_segments_s
   int64_t total = 0;
   std::vector<int64_t> offsets;  // nseg + 1, host copy
   int64_t* d_offsets = nullptr;
-  std::map<std::pair<int64_t, int64_t>, rs::TileTable> tables;  // (tile, short limit)
+  std::map<std::pair<int64_t, int64_t>, rs::TileTable> tables;  // scans: (tile, short limit)
+  std::map<int64_t, rs::ReduceTable> reduce_tables;             // quad elements
   // The segments as the batched sort takes them, built at the plan's first
   // sort: records of those one block sorts, by length class (rsort::
   // order_by_class), tile records of the longer ones (segmented onesweep) and
