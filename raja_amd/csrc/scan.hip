@@ -20,6 +20,7 @@
 //     need clearing between calls; under graph capture (where the epoch is
 //     frozen into the graph) a clear kernel runs first.
 #include <mutex>
+#include <optional>
 #include <type_traits>
 
 #include "ops.hpp"
@@ -57,50 +58,78 @@ struct ScanShape
       VO != 0 ? VO : (sizeof(T) == 8 ? 12 : (MODE == 0 ? 16 : (MODE == 1 ? 8 : 4)));
   static constexpr int WCHUNK = wave_size * V * VEC;   // elements per wave
   static constexpr int64_t TILE = (int64_t)kWaves * WCHUNK;
-  typedef T vec_t __attribute__((ext_vector_type(16 / sizeof(T))));
-  // The same 16 bytes at the element's own alignment: a tile of a segment
+  // 16 bytes at the element's own alignment: a tile of a segment or of a slice
   // starts at any element.  16-byte global accesses need only 4-byte
   // alignment on CDNA.
   typedef T uvec_t __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
 };
 
-// Elements [i0, i0 + VEC) of a lane's vector where only indices < n exist:
-// one 16-byte access when the whole vector is in range, element accesses at
-// the range's end.
+// The first `rem` elements of a wave's chunk at p (rem < WCHUNK), the identity
+// past them.  Lanes past the last whole vector load that one again and rows
+// past it load nothing, so the loads are unguarded 16-byte ones all in flight;
+// the up to VEC - 1 elements after it are their lane's own loads.  (A guarded
+// choice of vector or element loads per row: a one-tile span of 1000 int32
+// took 7.4 us, a full tile 4.6; the scan of 20,000 uneven segments 156 us
+// against 146 now, stores nontemporal as in full tiles.)
 template<typename S, typename T>
-__device__ __forceinline__ void load_vec_guarded(const T* in, int64_t i0, int64_t n,
-                                                 T (&v)[S::VEC], T ident)
+__device__ __forceinline__ void load_partial(const T* p, int rem, T (&v)[S::V][S::VEC], T ident)
 {
-  if (i0 + S::VEC <= n)
-  {
-    const typename S::uvec_t x = *reinterpret_cast<const typename S::uvec_t*>(in + i0);
+  constexpr int VEC = S::VEC;
+  const int lane = lane_id();
+  const int nv = rem / VEC;
+  T tail[VEC];
 #pragma unroll
-    for (int e = 0; e < S::VEC; ++e) v[e] = x[e];
+  for (int e = 0; e < VEC - 1; ++e)
+  {
+    tail[e] = (lane == nv % wave_size && nv * VEC + e < rem) ? p[nv * VEC + e] : ident;
   }
-  else
-  {
+  typename S::uvec_t x[S::V];
 #pragma unroll
-    for (int e = 0; e < S::VEC; ++e) v[e] = (i0 + e < n) ? in[i0 + e] : ident;
+  for (int k = 0; k < S::V; ++k)
+  {
+    const int q = k * wave_size + lane;
+    if (k * wave_size < nv)
+    {
+      x[k] = __builtin_nontemporal_load(
+          reinterpret_cast<const typename S::uvec_t*>(p + (q < nv ? q : nv - 1) * VEC));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < S::V; ++k)
+  {
+    const int q = k * wave_size + lane;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+    {
+      v[k][e] = (q < nv) ? x[k][e] : ((q == nv && e < VEC - 1) ? tail[e] : ident);
+    }
   }
 }
 
 template<typename S, typename T>
-__device__ __forceinline__ void store_vec_guarded(T* out, int64_t i0, int64_t n,
-                                                  const T (&o)[S::VEC])
+__device__ __forceinline__ void store_partial(T* p, int rem, const T (&o)[S::V][S::VEC])
 {
-  if (i0 + S::VEC <= n)
-  {
-    typename S::uvec_t x;
+  constexpr int VEC = S::VEC;
+  const int lane = lane_id();
+  const int nv = rem / VEC;
 #pragma unroll
-    for (int e = 0; e < S::VEC; ++e) x[e] = o[e];
-    *reinterpret_cast<typename S::uvec_t*>(out + i0) = x;
-  }
-  else
+  for (int k = 0; k < S::V; ++k)
   {
-#pragma unroll
-    for (int e = 0; e < S::VEC; ++e)
+    const int q = k * wave_size + lane;
+    if (q < nv)
     {
-      if (i0 + e < n) out[i0 + e] = o[e];
+      typename S::uvec_t x;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) x[e] = o[k][e];
+      __builtin_nontemporal_store(x, reinterpret_cast<typename S::uvec_t*>(p + q * VEC));
+    }
+    else if (q == nv)
+    {
+#pragma unroll
+      for (int e = 0; e < VEC - 1; ++e)
+      {
+        if (q * VEC + e < rem) p[q * VEC + e] = o[k][e];
+      }
     }
   }
 }
@@ -207,7 +236,7 @@ __device__ __forceinline__ T lookback(const Desc<T>* desc, int64_t tile, int64_t
 // MODE != 0 (SEG): the tiles of many ranges (segments) come from a tile
 // table; each range starts from `init` and its lookback stops at its own
 // first tile.
-template<typename T, typename Op, bool EXCLUSIVE, bool ALIGNED, int MODE, int VO = 0>
+template<typename T, typename Op, bool EXCLUSIVE, int MODE, int VO = 0>
 __global__ __launch_bounds__(kBlock) void scan_kernel(const T* in, T* out, int64_t n, T init,
                                                       Desc<T>* __restrict__ desc,
                                                       uint32_t epoch_tag,
@@ -215,7 +244,7 @@ __global__ __launch_bounds__(kBlock) void scan_kernel(const T* in, T* out, int64
 {
   constexpr bool SEG = MODE != 0;
   using S = ScanShape<T, MODE, VO>;
-  using vec_t = typename S::vec_t;
+  using lvec_t = typename S::uvec_t;
   constexpr int VEC = S::VEC;
   constexpr int V = S::V;
   const Op op{};
@@ -235,14 +264,13 @@ __global__ __launch_bounds__(kBlock) void scan_kernel(const T* in, T* out, int64
     out += r.out_delta;  // output element i of the range lands at out[i + out_delta]
   }
   const int lane = lane_id();
-  const int wave = wave_id();
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int64_t wbase = tbase + (int64_t)wave * S::WCHUNK;
-  // A segment's tiles start at any element: they take 16-byte accesses at the
-  // element's alignment.  A span's tiles take 16-byte aligned ones when the
-  // host found both pointers aligned.
-  using lvec_t = std::conditional_t<SEG, typename S::uvec_t, vec_t>;
-  const bool full = (SEG || ALIGNED) && tbase + S::TILE <= nend;
-  n = nend;
+  // Tiles start at any element (segments, slices): 16-byte accesses at the
+  // element's alignment.
+  const bool full = tbase + S::TILE <= nend;
+  const int64_t left = nend - wbase;  // elements of this wave's chunk
+  const int rem = left <= 0 ? 0 : (left < S::WCHUNK ? (int)left : S::WCHUNK);
 
   T v[V][VEC];
   if (full)
@@ -258,11 +286,7 @@ __global__ __launch_bounds__(kBlock) void scan_kernel(const T* in, T* out, int64
   }
   else
   {
-#pragma unroll
-    for (int k = 0; k < V; ++k)
-    {
-      load_vec_guarded<S>(in, wbase + ((int64_t)k * wave_size + lane) * VEC, n, v[k], Op::ident());
-    }
+    load_partial<S>(in + wbase, rem, v, Op::ident());
   }
 
   // Per-lane exclusive prefix of each vector within the wave's chunk.
@@ -348,11 +372,7 @@ __global__ __launch_bounds__(kBlock) void scan_kernel(const T* in, T* out, int64
   }
   else
   {
-#pragma unroll
-    for (int k = 0; k < V; ++k)
-    {
-      store_vec_guarded<S>(out, wbase + ((int64_t)k * wave_size + lane) * VEC, n, o[k]);
-    }
+    store_partial<S>(out + wbase, rem, o);
   }
 }
 
@@ -370,20 +390,13 @@ __global__ __launch_bounds__(kBlock) void short_scan_kernel(const T* __restrict_
   constexpr int VEC = S::VEC;
   constexpr int V = S::V;
   const Op op{};
-  const int64_t ri = (int64_t)blockIdx.x * kWaves + wave_id();
+  const int64_t ri = (int64_t)blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(wave_id());
   if (ri >= nrec) return;  // whole wave; the kernel has no barrier
   const rs::TileRec r = recs[ri];
-  const int lane = lane_id();
-  const int64_t b = r.seg_start;
-  const int64_t n = r.seg_start + r.seg_len;
-  T* const o_base = out + r.out_delta;
+  const int rem = (int)r.seg_len;
 
   T v[V][VEC];
-#pragma unroll
-  for (int k = 0; k < V; ++k)
-  {
-    load_vec_guarded<S>(in, b + ((int64_t)k * wave_size + lane) * VEC, n, v[k], Op::ident());
-  }
+  load_partial<S>(in + r.seg_start, rem, v, Op::ident());
   T lane_pref[V];
   T run = Op::ident();
 #pragma unroll
@@ -399,27 +412,27 @@ __global__ __launch_bounds__(kBlock) void short_scan_kernel(const T* __restrict_
   }
   const T start = EXCLUSIVE ? init : Op::ident();
   const T base_pref = op(start, Op::ident());
+  T o[V][VEC];
 #pragma unroll
   for (int k = 0; k < V; ++k)
   {
     T acc = op(base_pref, lane_pref[k]);
-    T o[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e)
     {
       if (EXCLUSIVE)
       {
-        o[e] = acc;
+        o[k][e] = acc;
         acc = op(acc, v[k][e]);
       }
       else
       {
         acc = op(acc, v[k][e]);
-        o[e] = acc;
+        o[k][e] = acc;
       }
     }
-    store_vec_guarded<S>(o_base, b + ((int64_t)k * wave_size + lane) * VEC, n, o);
   }
+  store_partial<S>(out + r.seg_start + r.out_delta, rem, o);
 }
 
 // Zero lookback descriptors (used only when the stream is being captured:
@@ -445,8 +458,8 @@ int table_mode(const raja_cdna4_segments_s* plan)
 // tiles); otherwise tile table records of shape `mode` (1 or 2).  desc holds
 // ntiles descriptors; with `clear` they are zeroed first (required whenever
 // the memory may hold this epoch tag from an earlier use).
-// Span tile of 4- and 8-byte values for a tuned vectors-per-lane choice
-// (0: the default shape).  The tuned shapes are taken by aligned spans.
+// Span tile of 4- and 8-byte values for a vectors-per-lane choice (0: the full
+// tile).
 template<typename T>
 constexpr int64_t span_tile(int v)
 {
@@ -458,15 +471,41 @@ constexpr int64_t span_tile(int v)
 template<typename T>
 constexpr int kSpanChoices[3] = {0, sizeof(T) == 8 ? 6 : 8, sizeof(T) == 8 ? 3 : 4};
 
+// Vectors per lane a span of n elements takes when nothing is tuned: one tile
+// (no lookback, no gate) in the smallest block that holds the span, then the
+// tile that gives the chip enough blocks, the full tile beyond.  Per call at
+// the full tile always / now, int32: n = 10007 10.3 / 4.4 us, 2^18 8.7 / 6.7,
+// 2^20 9.0 / 8.3, 2^21 10.9 / 9.4, 2^22 12.7 / 11.7; at 2^23 the full tile takes
+// 15.2 us against 18.3 with 4 vectors and 15.9 with 8.  int64: n = 1000 8.9 / 3.5,
+// 2^16 9.5 / 6.8, 2^18 9.7 / 7.9 (6 vectors; 8.1 with 3), 2^20 10.9 / 10.2; at
+// 2^21 the full tile 12.3 against 12.6 with 6.  FP64 sums keep the full tile:
+// a segment's scan and the same range's alone give the same bits.
+template<typename T, typename Op>
+int rule_choice(int64_t n)
+{
+  constexpr int small = kSpanChoices<T>[2], mid = kSpanChoices<T>[1];
+  if (std::is_same_v<T, double> && std::is_same_v<Op, rk::OpPlus<T>>) return 0;
+  if (n <= span_tile<T>(small)) return small;
+  if (n <= span_tile<T>(mid)) return mid;
+  if (n <= span_tile<T>(0)) return 0;
+  if (sizeof(T) == 4) return n <= 512 * span_tile<T>(small) ? small : 0;
+  if (n <= 64 * span_tile<T>(small)) return small;
+  return n <= 192 * span_tile<T>(mid) ? mid : 0;
+}
+
 template<typename T, typename Op, bool EXCLUSIVE>
 int launch_scan_core(const T* in, T* out, int64_t n, T init, hipStream_t s, const char* name,
                      const rs::TileRec* tiles, int64_t ntiles, void* desc, uint32_t epoch_tag,
                      bool clear, int mode = 1, int v = 0, bool gate_may_create = true)
 {
-  // one lookback launch at a time on the device (see rc::LookbackGate)
-  rc::LookbackGate gate(s, gate_may_create);
-  RC_TRY(gate.status());
-  const bool aligned = (((uintptr_t)in | (uintptr_t)out) % 16) == 0;
+  // one lookback launch at a time on the device (see rc::LookbackGate); a
+  // launch of one tile waits for no other block
+  std::optional<rc::LookbackGate> gate;
+  if (ntiles > 1)
+  {
+    gate.emplace(s, gate_may_create);
+    RC_TRY(gate->status());
+  }
   if (clear)
   {
     const int64_t words = ntiles * (int64_t)sizeof(Desc<T>) / 8;
@@ -474,12 +513,16 @@ int launch_scan_core(const T* in, T* out, int64_t n, T init, hipStream_t s, cons
                        dim3(256), 0, s, (uint64_t*)desc, words);
   }
   rc::TimedScope ts(name, s);
+  const dim3 grid((unsigned)ntiles), block(kBlock);
+  Desc<T>* const d = (Desc<T>*)desc;
+#define RSCAN_LAUNCH(MODE, V)                                                                      \
+  hipLaunchKernelGGL((scan_kernel<T, Op, EXCLUSIVE, MODE, V>), grid, block, 0, s, in, out, n, init, d, \
+                     epoch_tag, tiles)
   if (tiles && mode == 2)
   {
     if constexpr (sizeof(T) == 4)
     {
-      hipLaunchKernelGGL((scan_kernel<T, Op, EXCLUSIVE, false, 2>), dim3((unsigned)ntiles),
-                         dim3(kBlock), 0, s, in, out, n, init, (Desc<T>*)desc, epoch_tag, tiles);
+      RSCAN_LAUNCH(2, 0);
     }
     else
     {
@@ -487,34 +530,14 @@ int launch_scan_core(const T* in, T* out, int64_t n, T init, hipStream_t s, cons
     }
   }
   else if (tiles)
-  {
-    hipLaunchKernelGGL((scan_kernel<T, Op, EXCLUSIVE, false, 1>), dim3((unsigned)ntiles),
-                       dim3(kBlock), 0, s, in, out, n, init, (Desc<T>*)desc, epoch_tag, tiles);
-  }
-  else if (aligned && v == kSpanChoices<T>[1])
-  {
-    hipLaunchKernelGGL((scan_kernel<T, Op, EXCLUSIVE, true, 0, kSpanChoices<T>[1]>),
-                       dim3((unsigned)ntiles), dim3(kBlock), 0, s, in, out, n, init,
-                       (Desc<T>*)desc, epoch_tag, (const rs::TileRec*)nullptr);
-  }
-  else if (aligned && v == kSpanChoices<T>[2])
-  {
-    hipLaunchKernelGGL((scan_kernel<T, Op, EXCLUSIVE, true, 0, kSpanChoices<T>[2]>),
-                       dim3((unsigned)ntiles), dim3(kBlock), 0, s, in, out, n, init,
-                       (Desc<T>*)desc, epoch_tag, (const rs::TileRec*)nullptr);
-  }
-  else if (aligned)
-  {
-    hipLaunchKernelGGL((scan_kernel<T, Op, EXCLUSIVE, true, 0>), dim3((unsigned)ntiles),
-                       dim3(kBlock), 0, s, in, out, n, init, (Desc<T>*)desc, epoch_tag,
-                       (const rs::TileRec*)nullptr);
-  }
+    RSCAN_LAUNCH(1, 0);
+  else if (v == kSpanChoices<T>[1])
+    RSCAN_LAUNCH(0, kSpanChoices<T>[1]);
+  else if (v == kSpanChoices<T>[2])
+    RSCAN_LAUNCH(0, kSpanChoices<T>[2]);
   else
-  {
-    hipLaunchKernelGGL((scan_kernel<T, Op, EXCLUSIVE, false, 0>), dim3((unsigned)ntiles),
-                       dim3(kBlock), 0, s, in, out, n, init, (Desc<T>*)desc, epoch_tag,
-                       (const rs::TileRec*)nullptr);
-  }
+    RSCAN_LAUNCH(0, 0);
+#undef RSCAN_LAUNCH
   RC_HIP(hipGetLastError());
   return RAJA_CDNA4_SUCCESS;
 }
@@ -522,8 +545,8 @@ int launch_scan_core(const T* in, T* out, int64_t n, T init, hipStream_t s, cons
 // table == nullptr: one span of n elements; otherwise the tiles of a
 // segment plan (n = total elements of the plan).  Descriptors come from the
 // stream's scratch.
-// A span takes the tuned shape of its (kind, dtype, length bucket) when both
-// pointers are 16-byte aligned (v < 0: look it up; v >= 0: this shape).
+// A span takes the tuned shape of its (kind, dtype, length bucket), else that
+// of rule_choice (v < 0: look it up; v >= 0: this shape, 0 the rule's).
 template<typename T, typename Op, bool EXCLUSIVE>
 int launch_scan(const T* in, T* out, int64_t n, T init, hipStream_t s, const char* name,
                 const rs::TileTable* table = nullptr, int mode = 1, int v = -1)
@@ -532,7 +555,7 @@ int launch_scan(const T* in, T* out, int64_t n, T init, hipStream_t s, const cha
   if (n == 0) return RAJA_CDNA4_SUCCESS;  // empty range: no-op (pattern/scan.hpp:72-75)
   if (!in || !out) return rc::set_error(RAJA_CDNA4_ERROR_INVALID_ARGUMENT, "NULL span");
   int vv = 0;
-  if (!table && (((uintptr_t)in | (uintptr_t)out) % 16) == 0)
+  if (!table)
   {
     vv = v;
     if (vv < 0)
@@ -540,7 +563,7 @@ int launch_scan(const T* in, T* out, int64_t n, T init, hipStream_t s, const cha
       RC_TRY(rtune::choice(EXCLUSIVE ? rtune::kExclusiveScan : rtune::kInclusiveScan,
                            rk::dtype_code<T>(), n, s, &vv));
     }
-    if (vv != kSpanChoices<T>[1] && vv != kSpanChoices<T>[2]) vv = 0;
+    if (vv != kSpanChoices<T>[1] && vv != kSpanChoices<T>[2]) vv = rule_choice<T, Op>(n);
   }
   const int64_t ntiles = table ? table->ntiles : rc::ceil_div(n, span_tile<T>(vv));
   if (ntiles == 0) return RAJA_CDNA4_SUCCESS;
@@ -801,7 +824,8 @@ int noalloc_scratch(int dev, void** out)
 template<typename T, typename Op>
 int noalloc_scan_op(const T* in, T* out, int64_t n, T init, hipStream_t s, void* desc)
 {
-  const int64_t ntiles = rc::ceil_div(n, ScanShape<T>::TILE);
+  const int v = rule_choice<T, Op>(n);  // the shape (and FP bits) of the ordinary call
+  const int64_t ntiles = rc::ceil_div(n, span_tile<T>(v));
   if ((size_t)ntiles * sizeof(Desc<T>) > kNoAllocScratchBytes)
   {
     return rc::set_error(RAJA_CDNA4_ERROR_UNSUPPORTED,
@@ -814,7 +838,7 @@ int noalloc_scan_op(const T* in, T* out, int64_t n, T init, hipStream_t s, void*
   // memset, so the call can also be captured into a graph) zeroes them, and
   // the fixed tag 1 then marks this call's.  No timing events are created.
   return launch_scan_core<T, Op, true>(in, out, n, init, s, nullptr, nullptr, ntiles, desc,
-                                       1u << 2, true, 1, 0, /*gate_may_create=*/false);
+                                       1u << 2, true, 1, v, /*gate_may_create=*/false);
 }
 
 template<typename T>
