@@ -4,8 +4,11 @@ Headline workload: radix sort_pairs of N = 2^28 uint32 keys uniform over
 [0, 2^32) with int32 iota values (the sort configuration of the reference
 study).  One step = one sort_pairs call on resident inputs; the pristine keys
 and values are restored by a device copy before each step, outside the
-per-step event pair.  Algorithmic bytes per element = 16 per executed LSD
-pass (read+write key and value) + 4 for the digit-histogram read, P = 4.
+per-step event pair.  value counts 68 bytes per pair whichever way the sort
+runs: the four LSD passes of 8-bit digits (read+write key and value, 16 each)
+and the histogram read (4).  moves_executed and moved_bytes_per_elem say what
+this run moved: 16 per executed move (an LSD pass, or a scatter or the block
+sorts of the partition) + 4 for the histogram read.
 
 Also measured (reported under "ops"): the fused ReduceSum/Min/Max/MinLoc of
 N(0,1) FP64, exclusive_scan of int32 in [0,16), inclusive_scan of int64 and
@@ -127,15 +130,22 @@ def main():
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     R.timing_enable(False)
-    passes = R.timing_query("onesweep_pass")
-    hist = R.timing_query("radix_hist")
-    p_exec = passes["count"] // max(1, args.steps)
-    bytes_per_elem = 16 * p_exec + 4
+    # moves of the pairs (each reads and writes every pair once): LSD passes, or
+    # the scatters and block sorts of the partition
+    parts = [R.timing_query(k) for k in ("onesweep_pass", "partition_scatter", "partition_local")]
+    moves = sum(p["count"] for p in parts)
+    scatters = {k: sum(p[k] for p in parts[:2]) for k in ("count", "total_ms")}
+    hists = [R.timing_query(k) for k in ("radix_hist", "partition_sample", "partition_hist")]
+    hist = {"total_ms": sum(h["total_ms"] for h in hists), "count": args.steps}
+    passes = scatters
+    p_exec = moves // max(1, args.steps)
+    bytes_per_elem = 16 * 4 + 4
+    moved_per_elem = 16 * p_exec + 4
     ms = statistics.mean(step_ms)
     gbs = n * bytes_per_elem / (ms * 1e-3) / 1e9
     pass_ms = passes["total_ms"] / max(1, passes["count"])
     pass_gbs = n * 16 / (pass_ms * 1e-3) / 1e9
-    log("bench: sort_pairs %.3f ms/step (%.1f GB/s, %d passes), onesweep pass %.3f ms (%.1f GB/s)"
+    log("bench: sort_pairs %.3f ms/step (%.1f GB/s, %d moves), onesweep pass %.3f ms (%.1f GB/s)"
         % (ms, gbs, p_exec, pass_ms, pass_gbs))
 
     # correctness of the last step (size-independent, exact)
@@ -202,8 +212,9 @@ def main():
         "data": "synthetic (splitmix64 counter generator, seed 1; values iota)",
         "config": {
             "workload": "sort_pairs: N=2^%d uint32 keys uniform [0,2^32), int32 iota values, "
-                        "ascending, stable LSD onesweep 8-bit digits" % args.log2n,
-            "n": n, "passes_executed": p_exec, "bytes_per_elem": bytes_per_elem,
+                        "ascending, stable (two onesweep scatters and block sorts, or LSD onesweep 8-bit digits)" % args.log2n,
+            "n": n, "moves_executed": p_exec, "bytes_per_elem": bytes_per_elem,
+            "moved_bytes_per_elem": moved_per_elem, "moved_GB/s": round(n * moved_per_elem / (ms * 1e-3) / 1e9, 2),
             "hbm_frac": round(gbs / PEAK_GBS, 4), "keys_per_s": round(n / (ms * 1e-3), 1),
             "result_exact": ok, "wall_s_timed_loop": round(wall, 3),
         },

@@ -377,6 +377,7 @@ int raja_cdna4_stream_release(void* stream)
   if (c->tmp) RC_HIP(hipFree(c->tmp));
   if (c->pinned) RC_HIP(hipHostFree(c->pinned));
   if (c->small) RC_HIP(hipFree(c->small));
+  if (c->ready) RC_HIP(hipEventDestroy(c->ready));
   delete c;
   return RAJA_CDNA4_SUCCESS;
 }

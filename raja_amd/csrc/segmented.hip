@@ -284,9 +284,12 @@ int seg_sort(raja_cdna4_segments_s* p, K* keys, V* vals, int key_dtype, int val_
   RC_TRY(get_sort_table(p, &tab));
   if (tab->first[rsort::kLocalClasses] > 0)
   {
+    rc::StreamCtx* c = nullptr;
+    RC_TRY(rc::get_ctx(s, &c));
+    RC_TRY(rc::ensure_tmp(c, (size_t)tab->first[rsort::kLocalClasses] * sizeof(uint32_t)));
     rc::TimedScope ts("segmented_block_sort", s);
     RC_TRY(rsort::local_sort_batch(key_dtype, HAS_VALS ? val_bytes : 0, DESC ? 1 : 0, keys, vals, keys,
-                                   vals, tab->d_segs, tab->first, s));
+                                   vals, tab->d_segs, tab->first, (uint32_t*)c->tmp, s));
   }
   if (tab->longer.empty()) return RAJA_CDNA4_SUCCESS;
   if constexpr (sizeof(K) == 4 && (!HAS_VALS || sizeof(V) == 4))
@@ -373,12 +376,12 @@ int table_sum_f64(const double* base, const rs::TileRec* d_tiles, int64_t ntiles
 int64_t block_sort_max() { return rsort::local_sort_max(); }
 
 int block_sort_u32_i32(const uint32_t* base, const rs::SortSeg* d_segs,
-                       const int64_t (&first)[rsort::kLocalClasses + 1], hipStream_t s)
+                       const int64_t (&first)[rsort::kLocalClasses + 1], uint32_t* redo, hipStream_t s)
 {
   if (first[rsort::kLocalClasses] == 0) return RAJA_CDNA4_SUCCESS;
   rc::TimedScope ts("segmented_block_sort", s);
   return rsort::local_sort_batch(RAJA_CDNA4_U32, 4, 0, base, base, (void*)base, (void*)base, d_segs,
-                                 first, s);
+                                 first, redo, s);
 }
 }  // namespace rws
 

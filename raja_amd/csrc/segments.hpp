@@ -104,7 +104,7 @@ struct raja_cdna4_segments_s
   {
     bool built = false;
     rs::SortSeg* d_segs = nullptr;
-    int64_t first[5] = {0, 0, 0, 0, 0};
+    int64_t first[6] = {0, 0, 0, 0, 0, 0};
     rs::SortTile* d_tiles = nullptr;
     int64_t ntiles = 0;
     std::vector<int64_t> longer;

@@ -167,7 +167,7 @@ size_t batch_bytes_bound(const raja_cdna4_request& r)
     }
     default:
     {
-      if (r.n <= rws::block_sort_max()) return sizeof(rs::SortSeg);
+      if (r.n <= rws::block_sort_max()) return sizeof(rs::SortSeg) + sizeof(uint32_t);
       // segmented onesweep: records, descriptors, a histogram row and the
       // alternate keys and values
       const int64_t t = rc::ceil_div(r.n, rsort::seg_tile());
@@ -176,7 +176,7 @@ size_t batch_bytes_bound(const raja_cdna4_request& r)
     }
   }
 }
-constexpr size_t kBatchFixedBound = 6 * 16 + 8 * kAlign + 16;
+constexpr size_t kBatchFixedBound = 6 * 16 + 9 * kAlign + 16;
 
 // Host image of one batch: the records of each kind plus the layout of the
 // device copy (records first, then partials and descriptors).
@@ -192,7 +192,7 @@ struct BatchPlan
   uintptr_t sum_base = 0, scan_base = 0, sort_base = 0;
   size_t o_sum_tiles = 0, o_sum_first = 0, o_sum_count = 0, o_sum_out = 0, o_scan_tiles = 0,
          o_sorts = 0, o_sort_tiles = 0, rec_bytes = 0, o_partials = 0, o_desc = 0, o_sdesc = 0,
-         o_hist = 0, o_alt_k = 0, o_alt_v = 0, total = 0;
+         o_hist = 0, o_alt_k = 0, o_alt_v = 0, o_redo = 0, total = 0;
 
   void clear()
   {
@@ -307,6 +307,8 @@ struct BatchPlan
     o += rc::align_up((size_t)alt_elems * 4, kAlign);
     o_alt_v = o;
     o += rc::align_up((size_t)alt_elems * 4, kAlign);
+    o_redo = o;
+    o += rc::align_up(sorts.size() * sizeof(uint32_t), kAlign);
     total = o;
   }
 
@@ -421,7 +423,7 @@ int launch_batch(raja_cdna4_server_s* sv, Slot& slot, char* dev, hipStream_t s)
   {
     hipStream_t bs = side ? sv->upload : s;
     RC_TRY(rws::block_sort_u32_i32((const uint32_t*)p.sort_base, (const rs::SortSeg*)(dev + p.o_sorts),
-                                   p.sort_first, bs));
+                                   p.sort_first, (uint32_t*)(dev + p.o_redo), bs));
     if (side) RC_HIP(hipEventRecord(slot.sorted, bs));
   }
   if (!p.sum_out.empty())

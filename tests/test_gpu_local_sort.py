@@ -9,7 +9,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-EDGES = [1, 2, 63, 64, 65, 127, 128, 129, 255, 511, 512, 513, 1025, 2047, 2048, 2049, 5000, 8191, 8192]
+EDGES = [1, 2, 63, 64, 65, 127, 128, 129, 255, 511, 512, 513, 1025, 2047, 2048, 2049, 5000, 5119, 5120, 5121, 8191, 8192]
 TYPES = {"u32": np.uint32, "i32": np.int32, "f32": np.float32,
          "u64": np.uint64, "i64": np.int64, "f64": np.float64}
 TORCH = {"u32": torch.uint32, "u64": torch.uint64}
