@@ -158,6 +158,15 @@ def _check(status):
 _initialized = set()
 
 
+def _stream_of(dev):
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+# The current stream's handle without building a Stream object, where this
+# torch has it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _stream_of)
+
+
 def _prep(*tensors):
     """Validate GPU tensors and return the current stream handle."""
     dev = None
@@ -174,7 +183,7 @@ def _prep(*tensors):
     if dev not in _initialized:
         _check(lib().raja_cdna4_init(dev))
         _initialized.add(dev)
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return _raw_stream(dev)
 
 
 def device_status():
@@ -194,9 +203,15 @@ def _same_device(*tensors):
     """Every tensor (None skipped) on one device; the C entry points take raw
     pointers and no lengths beyond n, so this and the size checks below run
     before any call."""
-    devs = {t.device for t in tensors if t is not None}
-    if len(devs) > 1:
-        raise RajaError("tensors on different devices: %s" % sorted(str(d) for d in devs))
+    first = None
+    for t in tensors:
+        if t is None:
+            continue
+        if first is None:
+            first = t.device
+        elif t.device != first:
+            devs = {u.device for u in tensors if u is not None}
+            raise RajaError("tensors on different devices: %s" % sorted(str(d) for d in devs))
 
 
 def _check_out(out, dtype, numel, what="out"):
@@ -217,7 +232,32 @@ def _check_plan(plan, *tensors):
             raise RajaError("tensor on %s, plan on %s" % (t.device, want))
 
 
+# Plain Python numbers go to the library as ctypes scalars (a one-element torch
+# tensor per call cost about 3 us of a 10 us call); anything else, and numbers
+# outside the type's range, takes torch's conversion and its errors.
+_INT_SCALARS = {
+    torch.int32: (ctypes.c_int32, -(1 << 31), (1 << 31) - 1),
+    torch.int64: (ctypes.c_int64, -(1 << 63), (1 << 63) - 1),
+    torch.uint32: (ctypes.c_uint32, 0, (1 << 32) - 1),
+    torch.uint64: (ctypes.c_uint64, 0, (1 << 64) - 1),
+}
+_F32_MAX = 3.4028234663852886e38
+
+
 def _host_scalar(value, dtype):
+    t = type(value)
+    if t is int and dtype in _INT_SCALARS:
+        ctype, lo, hi = _INT_SCALARS[dtype]
+        if lo <= value <= hi:
+            c = ctype(value)
+            return c, ctypes.byref(c)
+    elif (t is float or (t is int and -(1 << 53) <= value <= 1 << 53)) and dtype.is_floating_point:
+        if dtype == torch.float64:
+            c = ctypes.c_double(value)
+            return c, ctypes.byref(c)
+        if dtype == torch.float32 and -_F32_MAX <= value <= _F32_MAX:
+            c = ctypes.c_float(value)
+            return c, ctypes.byref(c)
     buf = torch.tensor([value], dtype=dtype)
     return buf, ctypes.c_void_p(buf.data_ptr())
 
