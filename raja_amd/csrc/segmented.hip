@@ -21,12 +21,57 @@
 #include <string.h>
 
 #include <algorithm>
+#include <utility>
 #include <vector>
 
 #include "local_sort.hpp"
 #include "reduce_tree.hpp"
 #include "segments.hpp"
 #include "workspace.hpp"
+
+namespace
+{
+// A host array's copy on the device.  Freed again unless release() hands it
+// over, which a table's builder does once all its copies have succeeded: a
+// plan never holds an array whose upload failed (a first call under stream
+// capture is one way for it to fail).
+class Upload
+{
+ public:
+  Upload() = default;
+  Upload(const Upload&) = delete;
+  Upload& operator=(const Upload&) = delete;
+  ~Upload()
+  {
+    if (p_) (void)hipFree(p_);
+  }
+  template<typename T>
+  int put(const std::vector<T>& v)
+  {
+    const size_t bytes = sizeof(T) * v.size();
+    hipError_t e = hipMalloc(&p_, bytes ? bytes : 1);
+    if (e != hipSuccess)
+    {
+      p_ = nullptr;
+    }
+    else if (bytes)
+    {
+      e = hipMemcpy(p_, v.data(), bytes, hipMemcpyHostToDevice);
+    }
+    if (e == hipSuccess) return RAJA_CDNA4_SUCCESS;
+    (void)hipGetLastError();  // reported here, not by the next call's launch
+    return rc::hip_error(e, "segment table upload", __FILE__, __LINE__);
+  }
+  template<typename T>
+  T* release()
+  {
+    return static_cast<T*>(std::exchange(p_, nullptr));
+  }
+
+ private:
+  void* p_ = nullptr;
+};
+}  // namespace
 
 namespace rs
 {
@@ -54,16 +99,11 @@ int get_table(raja_cdna4_segments_s* p, int64_t tile, const TileTable** out, int
   }
   t.ntiles = (int64_t)recs.size();
   t.nshort = (int64_t)shorts.size();
-  RC_HIP(hipMalloc(&t.d_tiles, sizeof(TileRec) * (recs.size() + 1)));
-  RC_HIP(hipMalloc(&t.d_short, sizeof(TileRec) * (shorts.size() + 1)));
-  if (!recs.empty())
-  {
-    RC_HIP(hipMemcpy(t.d_tiles, recs.data(), sizeof(TileRec) * recs.size(), hipMemcpyHostToDevice));
-  }
-  if (!shorts.empty())
-  {
-    RC_HIP(hipMemcpy(t.d_short, shorts.data(), sizeof(TileRec) * shorts.size(), hipMemcpyHostToDevice));
-  }
+  Upload up_recs, up_shorts;
+  RC_TRY(up_recs.put(recs));
+  RC_TRY(up_shorts.put(shorts));
+  t.d_tiles = up_recs.release<TileRec>();
+  t.d_short = up_shorts.release<TileRec>();
   auto ins = p->tables.emplace(key, t);
   *out = &ins.first->second;
   return RAJA_CDNA4_SUCCESS;
@@ -174,8 +214,9 @@ int get_reduce_table(raja_cdna4_segments_s* p, int64_t quad, int64_t short_max, 
   image.reserve(sizeof(rs::TileRec) * (quads.size() + shorts.size()) + 16 * first.size() + 64);
   const size_t at_quads = place(quads), at_shorts = place(shorts), at_out = place(index),
                at_first = place(first), at_count = place(count);
-  RC_HIP(hipMalloc((void**)&t.mem, image.size() + 1));
-  if (!image.empty()) RC_HIP(hipMemcpy(t.mem, image.data(), image.size(), hipMemcpyHostToDevice));
+  Upload up;
+  RC_TRY(up.put(image));
+  t.mem = up.release<char>();
   t.d_quads = (const rs::TileRec*)(t.mem + at_quads);
   t.d_short = (const rs::TileRec*)(t.mem + at_shorts);
   t.d_out = (const int64_t*)(t.mem + at_out);
@@ -262,16 +303,11 @@ int get_sort_table(raja_cdna4_segments_s* p, const raja_cdna4_segments_s::SortTa
   }
   rsort::order_by_class(small, t.first);
   t.ntiles = (int64_t)recs.size();
-  if (!small.empty() && !t.d_segs)
-  {
-    RC_HIP(hipMalloc(&t.d_segs, sizeof(rs::SortSeg) * small.size()));
-    RC_HIP(hipMemcpy(t.d_segs, small.data(), sizeof(rs::SortSeg) * small.size(), hipMemcpyHostToDevice));
-  }
-  if (!recs.empty() && !t.d_tiles)
-  {
-    RC_HIP(hipMalloc(&t.d_tiles, sizeof(rs::SortTile) * recs.size()));
-    RC_HIP(hipMemcpy(t.d_tiles, recs.data(), sizeof(rs::SortTile) * recs.size(), hipMemcpyHostToDevice));
-  }
+  Upload up_segs, up_tiles;
+  if (!small.empty()) RC_TRY(up_segs.put(small));
+  if (!recs.empty()) RC_TRY(up_tiles.put(recs));
+  t.d_segs = up_segs.release<rs::SortSeg>();
+  t.d_tiles = up_tiles.release<rs::SortTile>();
   t.built = true;
   return RAJA_CDNA4_SUCCESS;
 }

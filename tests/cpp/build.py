@@ -46,7 +46,19 @@ def build_plugin():
     return out
 
 
+def build_host_paths():
+    """tests/cpp/bin/test_host_paths: the library's host code on a recording HIP
+    runtime, whose symbols the program exports to the library it loads."""
+    os.makedirs(BIN, exist_ok=True)
+    out = os.path.join(BIN, "test_host_paths")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I" + INC, "-I/opt/rocm/include",
+                    "-rdynamic", os.path.join(HERE, "test_host_paths.cpp"), "-o", out, "-ldl", "-lpthread"],
+                   check=True)
+    return out
+
+
 if __name__ == "__main__":
     print(build_host())
     print(build_gpu())
     print(build_plugin())
+    print(build_host_paths())

@@ -1,0 +1,30 @@
+"""Host code of the library on a recording HIP runtime (tests/cpp/
+recording_hip.hpp): launches, copies and waits in the order the calls make
+them, and calls that fail.  Runs without a GPU; no kernel runs."""
+import os
+import subprocess
+
+import pytest
+
+from tests.cpp import build as cppbuild
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "raja_amd", "libraja_cdna4.so")
+
+
+@pytest.fixture(scope="module")
+def exe():
+    return cppbuild.build_host_paths()
+
+
+def run(exe, name, tmp_path):
+    r = subprocess.run([exe, LIB, name], capture_output=True, text=True, timeout=120,
+                       env=dict(os.environ, RAJA_CDNA4_TUNE_DIR=str(tmp_path)))
+    print(r.stdout + r.stderr)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_plan_after_a_failed_upload(exe, tmp_path):
+    """A batched call whose table upload fails reports it and leaves the plan
+    as it was; the next call uploads the whole table."""
+    run(exe, "failed_upload", tmp_path)
