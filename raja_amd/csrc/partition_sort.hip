@@ -634,33 +634,40 @@ int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* a
     RC_HIP(hipGetLastError());
   }
   RC_HIP(hipEventRecord(ready, s));
-  rc::LookbackGate gate(s);  // one lookback launch at a time on the device
-  RC_TRY(gate.status());
   // The first scatter is launched before the decision is known here (it checks
-  // it on the device), so the wait below passes while it runs.
+  // it on the device), so the wait below passes while it runs.  The gate (one
+  // lookback launch at a time on the device) is held for each scatter's
+  // launch alone, never across the wait: other threads' scans and sorts
+  // must be able to go on, and this stream may be waiting for one of them.
   rs::SortTile* const recs = (rs::SortTile*)(aux + a.recs);
-  if (a.levels == 1)
   {
-    rc::TimedScope ts("partition_scatter", s);
-    launch_scatter<K, V, HAS_VALS, scatter_items(kb, vb, 1), 1>(keys, alt_k, vals, alt_v, n, plan, flip, count1, d0,
-                                                                d1, nullptr, a.ntiles, s);
+    rc::LookbackGate gate(s);
+    RC_TRY(gate.status());
+    if (a.levels == 1)
+    {
+      rc::TimedScope ts("partition_scatter", s);
+      launch_scatter<K, V, HAS_VALS, scatter_items(kb, vb, 1), 1>(keys, alt_k, vals, alt_v, n, plan, flip, count1, d0,
+                                                                  d1, nullptr, a.ntiles, s);
+    }
+    else
+    {
+      hipLaunchKernelGGL((records_kernel<K>), dim3(kRadix), dim3(256), 0, s, plan, (uint32_t*)(aux + a.rows),
+                         (uint32_t*)(aux + a.total), (uint32_t*)(aux + a.base), (uint32_t*)(aux + a.tile0),
+                         (uint32_t)a.tile, (uint32_t)n, window, (uint32_t)a.ngroups, recs, start, d1);
+      rc::TimedScope ts("partition_scatter", s);
+      launch_scatter<K, V, HAS_VALS, scatter_items(kb, vb, 2), 1>(keys, alt_k, vals, alt_v, n, plan, flip,
+                                                                  (uint32_t*)(aux + a.total), d0, d1, nullptr,
+                                                                  a.ntiles, s);
+    }
+    RC_HIP(hipGetLastError());
   }
-  else
-  {
-    hipLaunchKernelGGL((records_kernel<K>), dim3(kRadix), dim3(256), 0, s, plan, (uint32_t*)(aux + a.rows),
-                       (uint32_t*)(aux + a.total), (uint32_t*)(aux + a.base), (uint32_t*)(aux + a.tile0),
-                       (uint32_t)a.tile, (uint32_t)n, window, (uint32_t)a.ngroups, recs, start, d1);
-    rc::TimedScope ts("partition_scatter", s);
-    launch_scatter<K, V, HAS_VALS, scatter_items(kb, vb, 2), 1>(keys, alt_k, vals, alt_v, n, plan, flip,
-                                                                (uint32_t*)(aux + a.total), d0, d1, nullptr,
-                                                                a.ntiles, s);
-  }
-  RC_HIP(hipGetLastError());
   RC_HIP(hipEventSynchronize(ready));
   const uint32_t ok = *(volatile uint32_t*)host_ok;
   if (ok == 0u) return RAJA_CDNA4_SUCCESS;
   if (a.levels == 2)
   {
+    rc::LookbackGate gate(s);
+    RC_TRY(gate.status());
     rc::TimedScope ts("partition_scatter", s);
     launch_scatter<K, V, HAS_VALS, scatter_items(kb, vb, 2), 2>(alt_k, keys, alt_v, vals, n, plan, flip,
                                                                 (uint32_t*)(aux + a.rows), d1, d0, recs,

@@ -7,7 +7,12 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <chrono>
+#include <future>
+#include <memory>
 #include <string>
+#include <thread>
+#include <utility>
 #include <vector>
 
 #include "raja_cdna4.h"
@@ -107,6 +112,72 @@ void failed_upload()
     }
   }
 }
+
+// ---- the lookback gate -------------------------------------------------------------
+// What the partition's kernels leave in pinned memory when it takes the keys
+// (arguments as in partition_sort.hip).
+void take_partition(const std::string& kernel, void** args)
+{
+  if (kernel.find("sample_kernel") != std::string::npos) **(volatile uint32_t**)args[8] = 2u;
+  if (kernel.find("plan1_kernel") != std::string::npos) **(volatile uint32_t**)args[8] = 1u;
+  if (kernel.find("plan2_kernel") != std::string::npos) **(volatile uint32_t**)args[8] = 1u;
+}
+
+// While a sort waits on the host, a scan of many tiles on another thread and
+// stream must go through: the wait may be for work which that thread has yet
+// to queue.  And the gate's event covers the scatters alone: the block sorts,
+// which look back at nothing, are launched after it is recorded.
+void gate_across_waits()
+{
+  auto sort = ENTRY(raja_cdna4_sort_pairs);
+  auto scan = ENTRY(raja_cdna4_exclusive_scan);
+  hipStream_t s1 = nullptr, s2 = nullptr;
+  (void)hipStreamCreateWithFlags(&s1, 0);
+  (void)hipStreamCreateWithFlags(&s2, 0);
+  const int64_t n = 1 << 22;
+  std::vector<int32_t> in((size_t)n), out((size_t)n);
+  const int32_t zero = 0;
+  auto scan_on_s2 = [&] {
+    return scan(RAJA_CDNA4_I32, RAJA_CDNA4_OP_PLUS, in.data(), out.data(), n, &zero, s2);
+  };
+  CHECK(scan_on_s2() == 0, "scan");
+  for (const auto& [dtype, len] : {std::pair<int, int64_t>{RAJA_CDNA4_U32, 1 << 20}, {RAJA_CDNA4_U64, 1 << 22}})
+  {
+    std::vector<uint64_t> keys((size_t)len);
+    std::vector<uint32_t> vals((size_t)len);
+    rec::on_launch = take_partition;
+    CHECK(sort(dtype, keys.data(), vals.data(), 4, len, 0, s1) == 0, "sort");  // scratch
+    int waits = 0, stuck = 0;
+    std::thread::id me = std::this_thread::get_id();
+    rec::on_wait = [&](const char*) {
+      if (std::this_thread::get_id() != me) return;
+      ++waits;
+      auto done = std::make_shared<std::promise<int>>();
+      std::future<int> f = done->get_future();
+      std::thread([done, &scan_on_s2] { done->set_value(scan_on_s2()); }).detach();
+      if (f.wait_for(std::chrono::seconds(5)) != std::future_status::ready) ++stuck;
+    };
+    rec::clear();
+    CHECK(sort(dtype, keys.data(), vals.data(), 4, len, 0, s1) == 0, "sort");
+    rec::on_wait = nullptr;
+    CHECK(waits > 0, "the sort of %lld keys waits for nothing", (long long)len);
+    CHECK(stuck == 0, "a scan on another thread stood still while the sort waited");
+    if (stuck) std::this_thread::sleep_for(std::chrono::seconds(1));
+    rec::on_launch = nullptr;
+    std::lock_guard<std::recursive_mutex> g(rec::g_m);
+    size_t scatter = 0, recorded = 0, groups = 0;
+    for (size_t i = 0; i < rec::g_calls.size(); ++i)
+    {
+      const rec::Call& c = rec::g_calls[i];
+      if (c.stream != (void*)s1) continue;
+      if (c.kernel.find("onesweep_kernel") != std::string::npos) scatter = i;
+      if (c.kernel.find("local_groups_kernel") != std::string::npos) groups = i;
+      if (c.what == "event_record" && groups == 0) recorded = i;
+    }
+    CHECK(scatter > 0 && groups > scatter, "no partition");
+    CHECK(recorded > scatter, "the gate's event is recorded after the block sorts");
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -119,7 +190,8 @@ int main(int argc, char** argv)
     return 2;
   }
   if (ENTRY(raja_cdna4_init)(0) != 0) return 2;
-  const std::map<std::string, void (*)()> tests = {{"failed_upload", failed_upload}};
+  const std::map<std::string, void (*)()> tests = {{"failed_upload", failed_upload},
+                                                      {"gate_across_waits", gate_across_waits}};
   const auto it = tests.find(argv[2]);
   if (it == tests.end()) return 2;
   it->second();

@@ -28,3 +28,9 @@ def test_plan_after_a_failed_upload(exe, tmp_path):
     """A batched call whose table upload fails reports it and leaves the plan
     as it was; the next call uploads the whole table."""
     run(exe, "failed_upload", tmp_path)
+
+
+def test_lookback_gate_is_not_held_across_host_waits(exe, tmp_path):
+    """While a sort waits for its decision, scans on other threads and streams
+    go through; the gate's event covers the scatters, not the block sorts."""
+    run(exe, "gate_across_waits", tmp_path)
