@@ -587,7 +587,7 @@ __device__ __forceinline__ int items_of(int n)
 // The passes and the bin placement are kernels of their own where many ranges
 // are sorted: in one kernel the passes' registers make the placement spill
 // (2048-key ranges, 2^26 pairs: 0.24 ms apart, 0.99 ms together).  The
-// placement leaves a word per range that says whether it is left to do; one
+// placement leaves a byte per range that says whether it is left to do; one
 // launch of lsd_kernel does those.
 
 // One record per block; redo[b] = 1 where the range is left to the passes.
@@ -596,7 +596,7 @@ __device__ __forceinline__ int items_of(int n)
 template<typename K, typename V, bool HAS_VALS, int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK, (sizeof(K) == 4 && (!HAS_VALS || sizeof(V) == 4)) ? 8 : 4)
 void local_sort_kernel(const K* in_keys, const V* in_vals, K* out_keys, V* out_vals,
-                       const rs::SortSeg* __restrict__ segs, uint32_t* __restrict__ redo, bits_of<K> flip)
+                       const rs::SortSeg* __restrict__ segs, uint8_t* __restrict__ redo, bits_of<K> flip)
 {
   __shared__ LocalLds<K, V, HAS_VALS, BLOCK, ITEMS> s;
   rs::SortSeg sg = segs[blockIdx.x];
@@ -610,14 +610,14 @@ void local_sort_kernel(const K* in_keys, const V* in_vals, K* out_keys, V* out_v
   const bool done = local_sort_bins<K, V, HAS_VALS, BLOCK, ITEMS>(
       s, in_keys + sg.in_keys, HAS_VALS ? in_vals + sg.in_vals : nullptr, out_keys + sg.out_keys,
       HAS_VALS ? out_vals + sg.out_vals : nullptr, n, per, wbase, flip);
-  if (threadIdx.x == 0) redo[blockIdx.x] = done ? 0u : 1u;
+  if (threadIdx.x == 0) redo[blockIdx.x] = done ? 0 : 1;
 }
 
 // Groups of neighbouring buckets of a partitioned span.
 template<typename K, typename V, bool HAS_VALS, int BLOCK>
 __global__ __launch_bounds__(BLOCK, (sizeof(K) == 4 && (!HAS_VALS || sizeof(V) == 4)) ? 8 : 4)
 void local_groups_kernel(const K* in_keys, const V* in_vals, K* out_keys, V* out_vals,
-                         const uint32_t* __restrict__ start, uint32_t* __restrict__ redo, bits_of<K> flip)
+                         const uint32_t* __restrict__ start, uint8_t* __restrict__ redo, bits_of<K> flip)
 {
   __shared__ LocalLds<K, V, HAS_VALS, BLOCK, 8> s;
   const int64_t first = uniform((int64_t)start[blockIdx.x]);
@@ -631,7 +631,7 @@ void local_groups_kernel(const K* in_keys, const V* in_vals, K* out_keys, V* out
         s, in_keys + first, HAS_VALS ? in_vals + first : nullptr, out_keys + first,
         HAS_VALS ? out_vals + first : nullptr, n, per, wbase, flip);
   }
-  if (threadIdx.x == 0) redo[blockIdx.x] = done ? 0u : 1u;
+  if (threadIdx.x == 0) redo[blockIdx.x] = done ? 0 : 1;
 }
 
 // The ranges (records `segs`, or groups `start`) that redo marks, a
@@ -640,7 +640,7 @@ template<typename K, typename V, bool HAS_VALS>
 __global__ __launch_bounds__(1024) void lsd_kernel(const K* in_keys, const V* in_vals, K* out_keys, V* out_vals,
                                                    const rs::SortSeg* __restrict__ segs,
                                                    const uint32_t* __restrict__ start,
-                                                   const uint32_t* __restrict__ redo, int64_t count,
+                                                   const uint8_t* __restrict__ redo, int64_t count,
                                                    bits_of<K> flip)
 {
   __shared__ LocalLds<K, V, HAS_VALS, 1024, 8> s;
@@ -648,7 +648,7 @@ __global__ __launch_bounds__(1024) void lsd_kernel(const K* in_keys, const V* in
   for (int64_t base = blockIdx.x; base < count; base += (int64_t)gridDim.x * 1024)
   {
     const int64_t mine = base + (int64_t)threadIdx.x * gridDim.x;
-    const bool todo = mine < count && redo[mine] != 0u;
+    const bool todo = mine < count && redo[mine] != 0;
     if (__syncthreads_or(todo) == 0) continue;
     if (threadIdx.x == 0) s_n = 0u;
     __syncthreads();
@@ -700,7 +700,7 @@ constexpr int64_t kLsdBlocks = 512;
 
 template<typename K, typename V, bool HAS_VALS>
 int launch_groups(int descending, const void* ik, const void* iv, void* ok_, void* ov, const uint32_t* start,
-                  int64_t ngroups, int64_t cap, uint32_t* redo, hipStream_t s)
+                  int64_t ngroups, int64_t cap, uint8_t* redo, hipStream_t s)
 {
   const bits_of<K> flip = descending ? ~(bits_of<K>)0 : (bits_of<K>)0;
   if (cap <= rsort::kGroupCaps[0])
@@ -725,7 +725,7 @@ int launch_groups(int descending, const void* ik, const void* iv, void* ok_, voi
 // One span (d_segs nullptr) or the records of a batch.
 template<typename K, typename V, bool HAS_VALS>
 int launch_classes(const K* ik, const V* iv, K* ok, V* ov, bits_of<K> flip, const rs::SortSeg* d_segs,
-                   int64_t span, const int64_t* first, uint32_t* redo, hipStream_t s)
+                   int64_t span, const int64_t* first, uint8_t* redo, hipStream_t s)
 {
   if (!d_segs)
   {
@@ -781,7 +781,7 @@ int launch_classes(const K* ik, const V* iv, K* ok, V* ov, bits_of<K> flip, cons
 
 template<typename K>
 int launch_key(int val_bytes, int descending, const void* ik, const void* iv, void* ok, void* ov,
-               const rs::SortSeg* d_segs, int64_t span, const int64_t* first, uint32_t* redo, hipStream_t s)
+               const rs::SortSeg* d_segs, int64_t span, const int64_t* first, uint8_t* redo, hipStream_t s)
 {
   const bits_of<K> flip = descending ? ~(bits_of<K>)0 : (bits_of<K>)0;
   switch (val_bytes)
@@ -801,7 +801,7 @@ int launch_key(int val_bytes, int descending, const void* ik, const void* iv, vo
 }
 
 int launch_any(int key_dtype, int val_bytes, int descending, const void* ik, const void* iv, void* ok,
-               void* ov, const rs::SortSeg* d_segs, int64_t span, const int64_t* first, uint32_t* redo,
+               void* ov, const rs::SortSeg* d_segs, int64_t span, const int64_t* first, uint8_t* redo,
                hipStream_t s)
 {
   switch (key_dtype)
@@ -822,13 +822,13 @@ namespace rsort
 {
 int local_sort_batch(int key_dtype, int val_bytes, int descending, const void* in_k, const void* in_v,
                      void* out_k, void* out_v, const rs::SortSeg* d_segs,
-                     const int64_t (&first)[kLocalClasses + 1], uint32_t* redo, hipStream_t s)
+                     const int64_t (&first)[kLocalClasses + 1], uint8_t* redo, hipStream_t s)
 {
   return launch_any(key_dtype, val_bytes, descending, in_k, in_v, out_k, out_v, d_segs, 0, first, redo, s);
 }
 
 int local_sort_groups(int key_dtype, int val_bytes, int descending, const void* in_k, const void* in_v,
-                      void* out_k, void* out_v, const uint32_t* start, int64_t ngroups, int64_t cap, uint32_t* redo,
+                      void* out_k, void* out_v, const uint32_t* start, int64_t ngroups, int64_t cap, uint8_t* redo,
                       hipStream_t s)
 {
 #define RSORT_GROUPS(CODE, K)                                                                              \

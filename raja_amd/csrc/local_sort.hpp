@@ -43,19 +43,19 @@ inline void order_by_class(std::vector<rs::SortSeg>& segs, int64_t (&first)[kLoc
 
 // Sorts every range of a record array ordered by order_by_class (element
 // offsets from the given bases); a range may be sorted in place.  `redo` holds
-// a word per record (working memory of this call).
+// a byte per record (working memory of this call).
 int local_sort_batch(int key_dtype, int val_bytes, int descending, const void* in_k, const void* in_v,
                      void* out_k, void* out_v, const rs::SortSeg* d_segs,
-                     const int64_t (&first)[kLocalClasses + 1], uint32_t* redo, hipStream_t s);
+                     const int64_t (&first)[kLocalClasses + 1], uint8_t* redo, hipStream_t s);
 
 // Longest group of each of the two blocks local_sort_groups has (8 keys per thread).
 constexpr int kGroupCaps[2] = {2560, 5120};
 
 // Sorts every group [start[g], start[g + 1]) of a span, g < ngroups, one block
 // each (start on the device; none longer than cap, one of kGroupCaps).
-// `redo`: a word per group.
+// `redo`: a byte per group.
 int local_sort_groups(int key_dtype, int val_bytes, int descending, const void* in_k, const void* in_v,
-                      void* out_k, void* out_v, const uint32_t* start, int64_t ngroups, int64_t cap, uint32_t* redo,
+                      void* out_k, void* out_v, const uint32_t* start, int64_t ngroups, int64_t cap, uint8_t* redo,
                       hipStream_t s);
 
 // Sorts one span of 1 .. local_sort_max() keys.

@@ -521,7 +521,7 @@ struct Aux
     tile0 = place(kRadix * 4);
     rows = levels == 2 ? place((size_t)kFine * 4) : 0;
     start = place((size_t)(ngroups + 1) * 4);
-    redo = place((size_t)ngroups * 4);
+    redo = place((size_t)ngroups);
     recs = levels == 2 ? place((size_t)(ntiles + kRadix) * sizeof(rs::SortTile)) : 0;
     bytes = o;
   }
@@ -678,7 +678,7 @@ int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* a
   rc::TimedScope ts("partition_local", s);
   RC_TRY(rsort::local_sort_groups(dtype, vb, descending, from_alt ? alt_k : keys,
                                   from_alt ? (const void*)alt_v : (const void*)vals, keys, vals, start, a.ngroups,
-                                  rsort::kGroupCaps[ok - 1], (uint32_t*)(aux + a.redo), s));
+                                  rsort::kGroupCaps[ok - 1], (uint8_t*)(aux + a.redo), s));
   *done = true;
   return RAJA_CDNA4_SUCCESS;
 }

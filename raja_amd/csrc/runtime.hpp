@@ -53,7 +53,7 @@ struct StreamCtx
   void* tmp = nullptr;           // general temporaries (alt buffers, partials)
   size_t tmp_cap = 0;
   void* pinned = nullptr;        // 64 KiB pinned host staging
-  void* small = nullptr;         // 64 KiB device slots for per-call results
+  void* small = nullptr;         // 64 KiB device slots of fixed place: marks and results of one call
   hipEvent_t ready = nullptr;    // recorded where a sort's host decision is known
   uint32_t scan_epoch = 0;       // tag of the latest scan's lookback descriptors
 };

@@ -318,27 +318,42 @@ int seg_sort(raja_cdna4_segments_s* p, K* keys, V* vals, int key_dtype, int val_
 {
   const raja_cdna4_segments_s::SortTable* tab = nullptr;
   RC_TRY(get_sort_table(p, &tab));
+  if (tab->first[rsort::kLocalClasses] == 0 && tab->longer.empty()) return RAJA_CDNA4_SUCCESS;
+  rc::StreamCtx* c = nullptr;
+  RC_TRY(rc::get_ctx(s, &c));
+  // Scratch of the whole call before its first launch: growing it waits for
+  // the stream.
+  constexpr bool kOneSweep = sizeof(K) == 4 && (!HAS_VALS || sizeof(V) == 4);
+  const int64_t nranges = (int64_t)tab->longer.size();
+  const size_t kb = rc::align_up((size_t)p->total * sizeof(K), 256);
+  const size_t vb = HAS_VALS ? rc::align_up((size_t)p->total * sizeof(V), 256) : 0;
+  if (kOneSweep && nranges > 0)
+  {
+    RC_TRY(rc::ensure_tmp(c, std::max(kb + vb + rsort::seg_hist_bytes(nranges),
+                                      (size_t)tab->first[rsort::kLocalClasses])));
+    RC_TRY(rc::ensure_sort_desc(c, rsort::seg_desc_bytes(tab->ntiles)));
+  }
   if (tab->first[rsort::kLocalClasses] > 0)
   {
-    rc::StreamCtx* c = nullptr;
-    RC_TRY(rc::get_ctx(s, &c));
-    RC_TRY(rc::ensure_tmp(c, (size_t)tab->first[rsort::kLocalClasses] * sizeof(uint32_t)));
+    // The block sorts' marks, a byte per segment: in the stream's fixed slots
+    // while they fit (no growth, so a capture needs no call of the same size
+    // before it, and a graph keeps a pointer that never moves).
+    const size_t marks = (size_t)tab->first[rsort::kLocalClasses];
+    uint8_t* redo = (uint8_t*)c->small;
+    if (marks > rc::small_slot_bytes)
+    {
+      RC_TRY(rc::ensure_tmp(c, marks));
+      redo = (uint8_t*)c->tmp;
+    }
     rc::TimedScope ts("segmented_block_sort", s);
     RC_TRY(rsort::local_sort_batch(key_dtype, HAS_VALS ? val_bytes : 0, DESC ? 1 : 0, keys, vals, keys,
-                                   vals, tab->d_segs, tab->first, (uint32_t*)c->tmp, s));
+                                   vals, tab->d_segs, tab->first, redo, s));
   }
   if (tab->longer.empty()) return RAJA_CDNA4_SUCCESS;
-  if constexpr (sizeof(K) == 4 && (!HAS_VALS || sizeof(V) == 4))
+  if constexpr (kOneSweep)
   {
     // Every longer segment in one segmented onesweep: alternates, histograms
     // and descriptors from the stream's scratch.
-    const int64_t nranges = (int64_t)tab->longer.size();
-    rc::StreamCtx* c = nullptr;
-    RC_TRY(rc::get_ctx(s, &c));
-    const size_t kb = rc::align_up((size_t)p->total * sizeof(K), 256);
-    const size_t vb = HAS_VALS ? rc::align_up((size_t)p->total * sizeof(V), 256) : 0;
-    RC_TRY(rc::ensure_tmp(c, kb + vb + rsort::seg_hist_bytes(nranges)));
-    RC_TRY(rc::ensure_sort_desc(c, rsort::seg_desc_bytes(tab->ntiles)));
     char* tmp = (char*)c->tmp;
     return rsort::seg_sort_table(key_dtype, HAS_VALS ? 4 : 0, DESC ? 1 : 0, keys, vals, keys, vals,
                                  tmp, HAS_VALS ? (void*)(tmp + kb) : nullptr, tab->d_tiles,
@@ -412,7 +427,7 @@ int table_sum_f64(const double* base, const rs::TileRec* d_tiles, int64_t ntiles
 int64_t block_sort_max() { return rsort::local_sort_max(); }
 
 int block_sort_u32_i32(const uint32_t* base, const rs::SortSeg* d_segs,
-                       const int64_t (&first)[rsort::kLocalClasses + 1], uint32_t* redo, hipStream_t s)
+                       const int64_t (&first)[rsort::kLocalClasses + 1], uint8_t* redo, hipStream_t s)
 {
   if (first[rsort::kLocalClasses] == 0) return RAJA_CDNA4_SUCCESS;
   rc::TimedScope ts("segmented_block_sort", s);

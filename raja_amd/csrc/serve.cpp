@@ -167,7 +167,7 @@ size_t batch_bytes_bound(const raja_cdna4_request& r)
     }
     default:
     {
-      if (r.n <= rws::block_sort_max()) return sizeof(rs::SortSeg) + sizeof(uint32_t);
+      if (r.n <= rws::block_sort_max()) return sizeof(rs::SortSeg) + 1;
       // segmented onesweep: records, descriptors, a histogram row and the
       // alternate keys and values
       const int64_t t = rc::ceil_div(r.n, rsort::seg_tile());
@@ -308,7 +308,7 @@ struct BatchPlan
     o_alt_v = o;
     o += rc::align_up((size_t)alt_elems * 4, kAlign);
     o_redo = o;
-    o += rc::align_up(sorts.size() * sizeof(uint32_t), kAlign);
+    o += rc::align_up(sorts.size(), kAlign);
     total = o;
   }
 
@@ -423,7 +423,7 @@ int launch_batch(raja_cdna4_server_s* sv, Slot& slot, char* dev, hipStream_t s)
   {
     hipStream_t bs = side ? sv->upload : s;
     RC_TRY(rws::block_sort_u32_i32((const uint32_t*)p.sort_base, (const rs::SortSeg*)(dev + p.o_sorts),
-                                   p.sort_first, (uint32_t*)(dev + p.o_redo), bs));
+                                   p.sort_first, (uint8_t*)(dev + p.o_redo), bs));
     if (side) RC_HIP(hipEventRecord(slot.sorted, bs));
   }
   if (!p.sum_out.empty())

@@ -46,8 +46,8 @@ int table_exclusive_i32(const int32_t* in_base, int32_t* out_base, const rs::Til
 
 // Stable sorts of (uint32, int32) ranges of at most block_sort_max() pairs,
 // one block or wave each, by records ordered by rsort::order_by_class; redo
-// holds a word per record.
+// holds a byte per record.
 int64_t block_sort_max();
 int block_sort_u32_i32(const uint32_t* base, const rs::SortSeg* d_segs,
-                       const int64_t (&first)[rsort::kLocalClasses + 1], uint32_t* redo, hipStream_t s);
+                       const int64_t (&first)[rsort::kLocalClasses + 1], uint8_t* redo, hipStream_t s);
 }  // namespace rws

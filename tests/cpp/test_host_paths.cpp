@@ -178,6 +178,52 @@ void gate_across_waits()
     CHECK(recorded > scatter, "the gate's event is recorded after the block sorts");
   }
 }
+
+// ---- scratch of a batched sort ------------------------------------------------------
+// All of a call's scratch grows before its first launch (growing waits for the
+// stream), and a batch of short segments grows none: it can be captured on a
+// stream that has run something else.
+void batched_sort_scratch()
+{
+  auto create = ENTRY(raja_cdna4_segments_create);
+  auto sort = ENTRY(raja_cdna4_segmented_sort_pairs);
+  auto scan = ENTRY(raja_cdna4_exclusive_scan);
+  std::vector<int64_t> off = {0};
+  for (int g = 0; g < 3000; ++g) off.push_back(off.back() + 1 + 37 * g % 8192);
+  const int64_t nshort = (int64_t)off.size() - 1;
+  for (int g = 0; g < 40; ++g) off.push_back(off.back() + 100000);
+  std::vector<uint32_t> keys((size_t)off.back()), vals(keys.size());
+  raja_cdna4_segments_s *all = nullptr, *few = nullptr;
+  CHECK(create(off.data(), (int64_t)off.size() - 1, &all) == 0, "create");
+  CHECK(create(off.data(), nshort, &few) == 0, "create");
+  CHECK(sort(few, RAJA_CDNA4_U32, keys.data(), vals.data(), 4, 0, nullptr) == 0, "tables");
+  CHECK(sort(all, RAJA_CDNA4_U32, keys.data(), vals.data(), 4, 0, nullptr) == 0, "tables");
+  hipStream_t s1 = nullptr, s2 = nullptr;
+  (void)hipStreamCreateWithFlags(&s1, 0);
+  (void)hipStreamCreateWithFlags(&s2, 0);
+  // scratch that a call of another kind left small
+  CHECK(sort(few, RAJA_CDNA4_U32, keys.data(), vals.data(), 4, 0, s1) == 0, "sort");
+  rec::clear();
+  CHECK(sort(all, RAJA_CDNA4_U32, keys.data(), vals.data(), 4, 0, s1) == 0, "sort");
+  size_t launched = 0;
+  for (const rec::Call& c : rec::g_calls)
+  {
+    launched += c.what == "launch";
+    CHECK(launched == 0 || (c.what != "malloc" && c.what != "free" && c.what != "stream_wait"),
+          "%s after %zu launches", c.what.c_str(), launched);
+  }
+  CHECK(launched > 6, "launches");
+
+  std::vector<int32_t> in(100), out(100);
+  const int32_t zero = 0;
+  CHECK(scan(RAJA_CDNA4_I32, RAJA_CDNA4_OP_PLUS, in.data(), out.data(), 100, &zero, s2) == 0, "scan");
+  rec::g_capturing = true;
+  rec::clear();
+  CHECK(sort(few, RAJA_CDNA4_U32, keys.data(), vals.data(), 4, 0, s2) == 0, "captured sort");
+  CHECK(rec::count("malloc") + rec::count("free") + rec::count("stream_wait") + rec::count("copy") == 0,
+        "a captured sort of short segments grows the stream's scratch");
+  rec::g_capturing = false;
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -191,7 +237,8 @@ int main(int argc, char** argv)
   }
   if (ENTRY(raja_cdna4_init)(0) != 0) return 2;
   const std::map<std::string, void (*)()> tests = {{"failed_upload", failed_upload},
-                                                      {"gate_across_waits", gate_across_waits}};
+                                                      {"gate_across_waits", gate_across_waits},
+                                                      {"batched_sort_scratch", batched_sort_scratch}};
   const auto it = tests.find(argv[2]);
   if (it == tests.end()) return 2;
   it->second();

@@ -34,3 +34,9 @@ def test_lookback_gate_is_not_held_across_host_waits(exe, tmp_path):
     """While a sort waits for its decision, scans on other threads and streams
     go through; the gate's event covers the scatters, not the block sorts."""
     run(exe, "gate_across_waits", tmp_path)
+
+
+def test_batched_sort_grows_its_scratch_first(exe, tmp_path):
+    """A batched sort takes all its scratch before its first launch; one of
+    short segments takes none, so a capture needs no growth."""
+    run(exe, "batched_sort_scratch", tmp_path)
