@@ -499,9 +499,11 @@ int launch_scan_core(const T* in, T* out, int64_t n, T init, hipStream_t s, cons
                      bool clear, int mode = 1, int v = 0, bool gate_may_create = true)
 {
   // one lookback launch at a time on the device (see rc::LookbackGate); a
-  // launch of one tile waits for no other block
+  // launch of one tile waits for no other block, but the allocation-free scan
+  // (the one that may not create the gate) clears and writes descriptors that
+  // all streams of the device share
   std::optional<rc::LookbackGate> gate;
-  if (ntiles > 1)
+  if (ntiles > 1 || !gate_may_create)
   {
     gate.emplace(s, gate_may_create);
     RC_TRY(gate->status());

@@ -224,6 +224,27 @@ void batched_sort_scratch()
         "a captured sort of short segments grows the stream's scratch");
   rec::g_capturing = false;
 }
+
+// The allocation-free scan's descriptors are one array per device: calls on
+// different streams run one after the other, one-tile calls too.
+void noalloc_order()
+{
+  auto scan = ENTRY(raja_cdna4_exclusive_scan_noalloc);
+  hipStream_t s[2] = {nullptr, nullptr};
+  for (hipStream_t& x : s) (void)hipStreamCreateWithFlags(&x, 0);
+  const int32_t zero = 0;
+  std::vector<int32_t> in(200000), out(200000);
+  for (int64_t n : {1, 1000, 200000})
+  {
+    for (int i = 0; i < 4; ++i)
+    {
+      rec::clear();
+      CHECK(scan(RAJA_CDNA4_I32, RAJA_CDNA4_OP_PLUS, in.data(), out.data(), n, &zero, s[i % 2]) == 0, "scan");
+      CHECK(i == 0 || rec::count("wait_event") == 1, "n = %lld: no wait for the other stream's scan", (long long)n);
+      CHECK(rec::count("event_record") == 1, "n = %lld: the next stream has nothing to wait for", (long long)n);
+    }
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -238,7 +259,8 @@ int main(int argc, char** argv)
   if (ENTRY(raja_cdna4_init)(0) != 0) return 2;
   const std::map<std::string, void (*)()> tests = {{"failed_upload", failed_upload},
                                                       {"gate_across_waits", gate_across_waits},
-                                                      {"batched_sort_scratch", batched_sort_scratch}};
+                                                      {"batched_sort_scratch", batched_sort_scratch},
+                                                      {"noalloc_order", noalloc_order}};
   const auto it = tests.find(argv[2]);
   if (it == tests.end()) return 2;
   it->second();

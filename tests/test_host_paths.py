@@ -40,3 +40,8 @@ def test_batched_sort_grows_its_scratch_first(exe, tmp_path):
     """A batched sort takes all its scratch before its first launch; one of
     short segments takes none, so a capture needs no growth."""
     run(exe, "batched_sort_scratch", tmp_path)
+
+
+def test_allocation_free_scans_of_two_streams_are_ordered(exe, tmp_path):
+    """They share one descriptor array, whatever their length."""
+    run(exe, "noalloc_order", tmp_path)
