@@ -232,8 +232,9 @@ enum raja_cdna4_tune_op
  * bucket and rewrite the cache file.  Synchronous. */
 int raja_cdna4_autotune(int tune_op, int dtype, int64_t n, void* stream);
 
-/* The shape a call of (tune_op, dtype, n) takes: *choice 0 is the default
- * shape, else vectors per lane (scans) or keys per thread (sorts); *tuned is
+/* The tuned shape of (tune_op, dtype, n): *choice 0 is the full tile, else
+ * vectors per lane (scans) or keys per thread (sorts, where they run digit
+ * passes); untuned lengths take the library's own rule; *tuned is
  * 1 when the bucket has a recorded measurement. */
 int raja_cdna4_tune_query(int tune_op, int dtype, int64_t n, int* choice, int* tuned);
 

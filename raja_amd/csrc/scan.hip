@@ -548,7 +548,7 @@ int launch_scan_core(const T* in, T* out, int64_t n, T init, hipStream_t s, cons
 // segment plan (n = total elements of the plan).  Descriptors come from the
 // stream's scratch.
 // A span takes the tuned shape of its (kind, dtype, length bucket), else that
-// of rule_choice (v < 0: look it up; v >= 0: this shape, 0 the rule's).
+// of rule_choice (v < 0: look it up; v >= 0: this shape, 0 the full tile).
 template<typename T, typename Op, bool EXCLUSIVE>
 int launch_scan(const T* in, T* out, int64_t n, T init, hipStream_t s, const char* name,
                 const rs::TileTable* table = nullptr, int mode = 1, int v = -1)
@@ -565,7 +565,10 @@ int launch_scan(const T* in, T* out, int64_t n, T init, hipStream_t s, const cha
       RC_TRY(rtune::choice(EXCLUSIVE ? rtune::kExclusiveScan : rtune::kInclusiveScan,
                            rk::dtype_code<T>(), n, s, &vv));
     }
-    if (vv != kSpanChoices<T>[1] && vv != kSpanChoices<T>[2]) vv = rule_choice<T, Op>(n);
+    if (vv < 0)
+      vv = rule_choice<T, Op>(n);
+    else if (vv != kSpanChoices<T>[1] && vv != kSpanChoices<T>[2])
+      vv = 0;
   }
   const int64_t ntiles = table ? table->ntiles : rc::ceil_div(n, span_tile<T>(vv));
   if (ntiles == 0) return RAJA_CDNA4_SUCCESS;

@@ -455,8 +455,10 @@ int sort_core(const K* in_keys, const V* in_vals, K* keys, V* vals, int64_t n, h
   return RAJA_CDNA4_SUCCESS;
 }
 
-// In-place sort with the stream's scratch, in the tuned tile shape of its
-// (key type, length bucket) (items < 0: look it up; else this shape).
+// In-place sort with the stream's scratch.  items >= 0: LSD passes in this tile
+// (0: the full one), for the tuner.  items < 0: one block, the partition or LSD
+// passes, by length and keys, the passes in the tuned tile of their (key type,
+// length bucket), else the length's.
 template<typename K, typename V, bool HAS_VALS, bool DESC>
 int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
 {
@@ -465,7 +467,8 @@ int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
     return rc::set_error(RAJA_CDNA4_ERROR_UNSUPPORTED, "sort length %lld exceeds %lld",
                          (long long)n, (long long)kMaxSortN);
   }
-  if (n <= rsort::local_sort_max())
+  const bool lsd_only = items >= 0;
+  if (!lsd_only && n <= rsort::local_sort_max())
   {
     // One launch of one block (local_sort.hip) instead of a clear, a
     // histogram and a pass per digit over one tile.
@@ -474,12 +477,8 @@ int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
                                  vals, keys, vals, n, s);
   }
   using S = SortShape<K, V, HAS_VALS>;
+  if (!lsd_only && !S::wide) RC_TRY(rtune::choice(rtune::kSortPairs, rk::dtype_code<K>(), n, s, &items));
   if (items < 0)
-  {
-    items = 0;
-    if (!S::wide) RC_TRY(rtune::choice(rtune::kSortPairs, rk::dtype_code<K>(), n, s, &items));
-  }
-  if (items <= 0 || (items != S::kChoices[1] && items != S::kChoices[2]))
   {
     // Untuned spans: small tiles where the full one leaves CUs idle.  FP32
     // keys ~ N(0, 1), per sort at 16384- / 8192- / 4096-key tiles: n = 10^4 93 /
@@ -496,7 +495,7 @@ int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
   RC_HIP(hipStreamIsCapturing(s, &cap));
   uint32_t* const pinned = cap == hipStreamCaptureStatusNone ? (uint32_t*)c->pinned : nullptr;
   constexpr int kb = (int)sizeof(K), vb = HAS_VALS ? (int)sizeof(V) : 0;
-  const bool part = pinned && rsort::partition_levels(kb, vb, n) > 0;
+  const bool part = !lsd_only && pinned && rsort::partition_levels(kb, vb, n) > 0;
   size_t tmp = w.tmp_bytes(), desc = w.desc_bytes;
   if (part)
   {

@@ -316,7 +316,7 @@ int bucket(int64_t n)
 
 int choice(int op, int dtype, int64_t n, hipStream_t s, int* out)
 {
-  *out = 0;
+  *out = kUntuned;
   if (!valid_op(op) || !valid_dtype(dtype) || n <= 0) return RAJA_CDNA4_SUCCESS;
   int dev = 0;
   RC_TRY(current_device(&dev));

@@ -29,9 +29,11 @@ enum Op
 // Length bucket of n: ceil(log2 n), at least 10.
 int bucket(int64_t n);
 
-// The shape a call of (op, dtype, n) takes: 0 for the default, else the
-// tuned candidate.  With RAJA_CDNA4_AUTOTUNE=1 in the environment an
-// untuned bucket is measured first (never while `s` is being captured).
+// The tuned shape of (op, dtype, n): a candidate (0: the full tile), or
+// kUntuned, which leaves the shape to the caller's rule on lengths.  With
+// RAJA_CDNA4_AUTOTUNE=1 in the environment an untuned bucket is measured first
+// (never while `s` is being captured).
+constexpr int kUntuned = -1;
 int choice(int op, int dtype, int64_t n, hipStream_t s, int* out);
 }  // namespace rtune
 

@@ -245,6 +245,65 @@ void noalloc_order()
     }
   }
 }
+
+// ---- shape tuning --------------------------------------------------------------------
+// The tuner's candidates run the kernels that they name, and a recorded full
+// tile is taken, not the tile that untuned spans of that length take.
+void tuner_shapes()
+{
+  auto tune = ENTRY(raja_cdna4_autotune);
+  auto forget = ENTRY(raja_cdna4_tune_forget);
+  auto path = ENTRY(raja_cdna4_tune_cache_path);
+  auto sort = ENTRY(raja_cdna4_sort_pairs);
+  auto scan = ENTRY(raja_cdna4_exclusive_scan);
+  auto shapes = [](const char* kernel) {  // grid sizes of a kernel's launches
+    std::set<unsigned> g;
+    for (const rec::Call& c : rec::g_calls)
+      if (c.kernel.find(kernel) != std::string::npos) g.insert(c.grid);
+    return g;
+  };
+  rec::on_launch = take_partition;
+  for (int64_t n : {int64_t(5000), int64_t(100000), int64_t(1) << 20})
+  {
+    rec::clear();
+    CHECK(tune(2, RAJA_CDNA4_U32, n, nullptr) == 0, "tune");
+    const std::set<unsigned> want = {(unsigned)((n + 16383) / 16384), (unsigned)((n + 8191) / 8192),
+                                     (unsigned)((n + 4095) / 4096)};
+    CHECK(shapes("onesweep_kernel") == want, "n = %lld: %zu tiles measured", (long long)n,
+          shapes("onesweep_kernel").size());
+    CHECK(rec::count("launch", "sample_kernel") + rec::count("launch", "span_sort_kernel") == 0,
+          "n = %lld: not the digit passes", (long long)n);
+  }
+  rec::on_launch = nullptr;  // pinned memory stays 0: the partition refuses
+  rec::clear();
+  CHECK(tune(1, RAJA_CDNA4_I32, 1 << 20, nullptr) == 0, "tune");
+  CHECK(shapes("scan_kernel") == (std::set<unsigned>{32, 64, 128}), "%zu scan tiles measured",
+        shapes("scan_kernel").size());
+
+  char file[1024];
+  CHECK(path(file, sizeof(file)) == 0, "path");
+  FILE* f = fopen(file, "w");
+  CHECK(f != nullptr, "%s", file);
+  if (!f) return;
+  fprintf(f, "sort_pairs 2 20 0 0.0\nexclusive_scan 0 20 0 0.0\n");
+  fclose(f);
+  std::vector<uint32_t> a(1 << 20), b(1 << 20);
+  const int32_t zero = 0;
+  for (int tuned = 1; tuned >= 0; --tuned)
+  {
+    CHECK(forget() == 0, "forget");
+    if (!tuned) remove(file);
+    rec::clear();
+    CHECK(sort(RAJA_CDNA4_U32, a.data(), b.data(), 4, 1 << 20, 0, nullptr) == 0, "sort");
+    // the partition's refused scatter has the small tile: count the digit passes' grid
+    size_t full = 0;
+    for (const rec::Call& c : rec::g_calls) full += c.kernel.find("onesweep_kernel") != std::string::npos && c.grid == 64;
+    CHECK((full > 0) == (tuned == 1), "full radix tile %s", tuned ? "not taken" : "taken untuned");
+    rec::clear();
+    CHECK(scan(RAJA_CDNA4_I32, RAJA_CDNA4_OP_PLUS, a.data(), b.data(), 1 << 20, &zero, nullptr) == 0, "scan");
+    CHECK(shapes("scan_kernel") == std::set<unsigned>{tuned ? 32u : 128u}, "scan tile");
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -260,7 +319,8 @@ int main(int argc, char** argv)
   const std::map<std::string, void (*)()> tests = {{"failed_upload", failed_upload},
                                                       {"gate_across_waits", gate_across_waits},
                                                       {"batched_sort_scratch", batched_sort_scratch},
-                                                      {"noalloc_order", noalloc_order}};
+                                                      {"noalloc_order", noalloc_order},
+                                                      {"tuner_shapes", tuner_shapes}};
   const auto it = tests.find(argv[2]);
   if (it == tests.end()) return 2;
   it->second();

@@ -43,8 +43,9 @@ def _sort(raja, k0, v0):
     return k.view(torch.int32).cpu().numpy().view(np.uint32), v.cpu().numpy()
 
 
-def test_cold_measured_warm_deleted_give_same_bits(raja, orc, tune_dir):
-    n = (1 << 20) + 77
+# sorts of 2^20 + 77 keys take the partition, of 2^21 + 77 the digit passes
+@pytest.mark.parametrize("n", [(1 << 20) + 77, (1 << 21) + 77])
+def test_cold_measured_warm_deleted_give_same_bits(raja, orc, tune_dir, n):
     x = torch.empty(n, dtype=torch.int32, device=DEV)
     raja.fill(raja.FILL_I32, x, seed=5, a=-50, b=50)
     want = orc.seq_exclusive(x.cpu().numpy(), orc.PLUS, 3)
@@ -86,7 +87,7 @@ def test_cold_measured_warm_deleted_give_same_bits(raja, orc, tune_dir):
     assert np.array_equal(_scan(raja, x, True), cold_scan)
 
 
-@pytest.mark.parametrize("dtype,choices", [(torch.int32, (8, 4)), (torch.int64, (6, 3))])
+@pytest.mark.parametrize("dtype,choices", [(torch.int32, (8, 4, 0)), (torch.int64, (6, 3, 0))])
 def test_every_scan_shape_exact(raja, orc, tune_dir, dtype, choices):
     n = 3_000_001
     x = torch.empty(n, dtype=dtype, device=DEV)
@@ -117,7 +118,7 @@ def test_every_sort_shape_exact(raja, orc, tune_dir, n):
                                        np.arange(n, dtype=np.int32))
     path = raja.tune_cache_path()
     b = int(np.ceil(np.log2(n)))
-    for c in (16, 8):
+    for c in (16, 8, 0):
         with open(path, "w") as f:
             f.write("sort_pairs 2 %d %d 0.0\n" % (b, c))
         raja.tune_forget()

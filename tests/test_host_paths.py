@@ -45,3 +45,9 @@ def test_batched_sort_grows_its_scratch_first(exe, tmp_path):
 def test_allocation_free_scans_of_two_streams_are_ordered(exe, tmp_path):
     """They share one descriptor array, whatever their length."""
     run(exe, "noalloc_order", tmp_path)
+
+
+def test_tuner_measures_and_takes_the_shapes_it_names(exe, tmp_path):
+    """Each candidate runs its own tile (digit passes for sorts, whatever the
+    keys), and a recorded full tile is the full tile."""
+    run(exe, "tuner_shapes", tmp_path)
