@@ -15,7 +15,16 @@
 // A sample of 4096 keys (one small kernel) rejects most other key sets; the
 // exact bucket counts decide before anything is moved; the first scatter checks
 // that decision on the device, so the host launches it without waiting, reads
-// the decision while it runs and goes on, or runs the LSD sort instead.
+// the decision while it runs and goes on, or runs the LSD sort instead.  Where
+// the sample refuses, the LSD sort's digit counts come next on the device and
+// the host is told which digits differ by a word in pinned memory (it used to
+// start over: clear, count, copy the histograms back, wait).  Refused spans,
+// LSD alone as it was before there was a partition / starting over / now: 16
+// distinct u32 keys and 4-byte values 2^20 70 / 83 / 64 us, 2^25 288 / 309 / 296;
+// 2^12 distinct 2^25 331 / 350 / 337; FP32 ~ N(0, 1) 2^20 137 / 134 / 109, 2^25 617 /
+// 638 / 624; FP64 ~ N(0, 1) and 4-byte values 2^20 199 / 214 / 196, 2^24 892 / 914 /
+// 899 us: one level no longer loses by being asked, two levels lose 5 to 8 us,
+// the sample.
 //
 // Per sort of uniform keys, LSD before / now: u32 keys and 4-byte values 2^18 109 /
 // 47 us, 2^20 127 / 63, 2^25 607 / 550, 2^28 4.07 / 3.50 ms (counts 0.20, scatters 1.00
@@ -24,6 +33,7 @@
 // are bound by vector instructions (about 160 per 64 keys).
 #include "partition_sort.hpp"
 
+#include "digit_hist.hpp"
 #include "key_map.hpp"
 #include "local_sort.hpp"
 #include "onesweep.hpp"
@@ -113,12 +123,16 @@ struct MapDigit
 // One block: range of the sampled keys, a little extended so that keys just
 // outside do not pile up in the end buckets, and whether the fullest of 256
 // equal parts of the range holds at most `most` samples and the range is at
-// least `least` wide.  Clears count1.
+// least `least` wide.  Few integer values: whether the values that share a bucket
+// (of per_bucket of the map's fine ones) fit into `bucket_most` keys if all
+// occur as often.  Clears count1 and the LSD sort's digit counters.
 template<typename K>
 __global__ __launch_bounds__(1024) void sample_kernel(const K* __restrict__ keys, int64_t n,
                                                       bits_of<K> flip, uint32_t most,
                                                       bits_of<K> least, Plan<K>* __restrict__ plan,
-                                                      uint32_t* __restrict__ count1, uint32_t tail_most,
+                                                      uint32_t* __restrict__ count1,
+                                                      uint32_t* __restrict__ lsd_hist, uint32_t per_bucket,
+                                                      uint32_t bucket_most,
                                                       uint32_t* host_word)
 {
   using bits_t = bits_of<K>;
@@ -139,6 +153,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(const K* __restrict__ keys
   }
   if (tid < kSampleBins) s_bin[tid] = 0u;
   if (tid < kRadix) count1[tid] = 0u;
+  for (int i = tid; i < (int)sizeof(K) * kRadix; i += 1024) lsd_hist[i] = 0u;
   bits_t lo = ~(bits_t)0, hi = 0;
 #pragma unroll
   for (int j = 0; j < PER; ++j)
@@ -160,6 +175,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(const K* __restrict__ keys
     lo = s_lo[w] < lo ? s_lo[w] : lo;
     hi = s_hi[w] > hi ? s_hi[w] : hi;
   }
+  const bits_t spread = hi - lo;
   // 8 sample gaps of a uniform key set on both sides
   bool ok = hi - lo >= least;
   if constexpr (std::is_floating_point_v<K>)
@@ -188,6 +204,14 @@ __global__ __launch_bounds__(1024) void sample_kernel(const K* __restrict__ keys
   p.hi = hi;
   const FineMap<K> fine(&p, flip);
   ok = ok && fine.bins.ok && lo < hi;
+  if constexpr (!std::is_floating_point_v<K>)
+  {
+    if (ok && fine.bins.scale == 0u)  // fewer values than fine buckets
+    {
+      const uint64_t share = (per_bucket - 1u) / fine.bins.mul + 1u;
+      ok = (uint64_t)n * share <= (uint64_t)bucket_most * ((uint64_t)spread + 1u);
+    }
+  }
   if (ok)
   {
 #pragma unroll
@@ -198,7 +222,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(const K* __restrict__ keys
   // A thin end means a tail that goes on past the sample's extremes: the end
   // bucket takes about one key in kSample.
   const bool tail = s_bin[0] < 2u || s_bin[kSampleBins - 1] < 2u;
-  ok = ok && !too_many && !(tail && n / kSample > (int64_t)tail_most);
+  ok = ok && !too_many && !(tail && n / kSample > (int64_t)bucket_most);
   if (tid == 0)
   {
     plan->lo = lo;
@@ -214,19 +238,28 @@ __global__ __launch_bounds__(1024) void sample_kernel(const K* __restrict__ keys
 // ---- one level: counts of the high byte --------------------------------------------------
 constexpr int kHist1Keys = 256 * 16;  // keys per block and step
 
+// Where the sample has refused the span: the LSD sort's digit counts instead, and
+// its descriptors.
 template<typename K>
 __global__ __launch_bounds__(256) void hist1_kernel(const K* __restrict__ keys, int64_t n,
                                                     bits_of<K> flip, const Plan<K>* __restrict__ plan,
                                                     uint32_t* __restrict__ count1,
-                                                    uint32_t* __restrict__ desc0, int64_t desc0_words)
+                                                    uint32_t* __restrict__ desc0, int64_t desc0_words,
+                                                    uint32_t* __restrict__ lsd_hist, int64_t lsd_desc_words)
 {
-  constexpr int kCopies = 8;
+  constexpr int kCopies = kHistCopies;
   constexpr int VEC = 16 / sizeof(K);
   constexpr int U = 16 / VEC;
   typedef K uvec_t __attribute__((ext_vector_type(16 / sizeof(K)), aligned(sizeof(K))));
-  if (!plan->sample_ok) return;
-  __shared__ uint32_t s_hist[kRadix * kCopies];
+  __shared__ uint32_t s_hist[kHistWords<K>];
   const int tid = threadIdx.x;
+  if (!plan->sample_ok)
+  {
+    count_digits<K>(keys, n, s_hist);
+    add_digits<K>(s_hist, lsd_hist, flip != 0);
+    for (int64_t i = (int64_t)blockIdx.x * 256 + tid; i < lsd_desc_words; i += (int64_t)gridDim.x * 256) desc0[i] = 0u;
+    return;
+  }
   for (int i = tid; i < kRadix * kCopies; i += 256) s_hist[i] = 0u;
   const FineMap<K> fine(plan, flip);
   __syncthreads();
@@ -290,18 +323,29 @@ template<typename K>
 __global__ __launch_bounds__(256) void plan1_kernel(Plan<K>* __restrict__ plan,
                                                     const uint32_t* __restrict__ count1, uint32_t n,
                                                     uint32_t most0, uint32_t most1, uint32_t window, uint32_t ngroups,
-                                                    uint32_t* __restrict__ start, uint32_t* host_ok)
+                                                    uint32_t* __restrict__ start,
+                                                    const uint32_t* __restrict__ lsd_hist, uint32_t* host)
 {
   __shared__ uint32_t s_w[4];
   const int t = threadIdx.x;
+  if (!plan->sample_ok)
+  {
+    const uint32_t digits = active_digits<K>(lsd_hist, n);
+    if (t == 0)
+    {
+      host[0] = 0u;
+      host[2] = digits;
+    }
+    return;
+  }
   const uint32_t c = count1[t];
   const bool small = __syncthreads_or(c > most0) == 0;
-  const bool ok = __syncthreads_or(c > most1) == 0 && plan->sample_ok;
+  const bool ok = __syncthreads_or(c > most1) == 0;
   if (t == 0)
   {
     const uint32_t v = ok ? (small ? 1u : 2u) : 0u;
     plan->ok = v;
-    *host_ok = v;
+    host[0] = v;
   }
   if (!ok) return;
   const uint32_t off = scan256(c, s_w);
@@ -566,9 +610,12 @@ void launch_scatter(const K* ik, K* ok, const V* iv, V* ov, int64_t n, const Pla
 }
 
 template<typename K, typename V, bool HAS_VALS>
-int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* alt_k, V* alt_v, char* aux,
-                    uint32_t* desc, uint32_t* host_ok, hipEvent_t ready, hipStream_t s, bool* done)
+int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, const rsort::PartitionMem& mem,
+                    hipStream_t s, bool* done, uint32_t* digits)
 {
+  K* const alt_k = (K*)mem.alt_keys;
+  V* const alt_v = (V*)mem.alt_vals;
+  char* const aux = mem.aux;
   constexpr int kb = (int)sizeof(K), vb = HAS_VALS ? (int)sizeof(V) : 0;
   const bits_of<K> flip = descending ? ~(bits_of<K>)0 : (bits_of<K>)0;
   const Aux a(kb, vb, n);
@@ -580,29 +627,40 @@ int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* a
   Plan<K>* const plan = (Plan<K>*)(aux + a.plan);
   uint32_t* const count1 = (uint32_t*)(aux + a.count1);
   uint32_t* const start = (uint32_t*)(aux + a.start);
-  uint32_t* const d0 = desc;
-  uint32_t* const d1 = desc + (a.ntiles + kRadix) * kRowStride;
+  uint32_t* const d0 = mem.desc;
+  uint32_t* const d1 = mem.desc + (a.ntiles + kRadix) * kRowStride;
+  volatile uint32_t* const host = mem.host;
+  host[0] = host[1] = host[2] = 0u;
   {
-    // Two levels: the host polls the sample's answer (a rejected span then costs
-    // one small kernel and no wait beyond it: about 13 us).  One level goes on
-    // without it: the wait would cost an accepted span as much as the kernels
-    // that end at once cost a rejected one (2^20 pairs: 63 against 75 us, 82
-    // against 77 for 16 distinct keys).
     rc::TimedScope ts("partition_sample", s);
-    volatile uint32_t* const word = host_ok + 1;
-    *word = 0u;
     hipLaunchKernelGGL((sample_kernel<K>), dim3(1), dim3(1024), 0, s, keys, n, flip,
-                       sample_limit(kb, n, a.levels), least, plan, count1, most1, host_ok + 1);
+                       sample_limit(kb, n, a.levels), least, plan, count1, mem.hist,
+                       (uint32_t)(kFine / buckets_of(a.levels)), most1, mem.host + 1);
     RC_HIP(hipGetLastError());
-    for (uint32_t polls = 1; a.levels == 2 && *word == 0u; ++polls)
+  }
+  // A span that the sample refuses has its digits counted by the kernel that
+  // follows, so it pays for the sample and little else.  One level: the counts'
+  // kernel does it, and the host goes on without the answer (a wait here
+  // would cost an accepted span as much as the kernels that end at once
+  // cost a refused one: 2^20 pairs 63 against 75 us).  Two levels: a kernel of its own,
+  // which ends at once where the span is accepted, while the host polls the answer.
+  if (a.levels == 2)
+  {
     {
-      if ((polls & 0xFFFu) != 0u) continue;
-      const hipError_t e = hipStreamQuery(s);  // a failed stream never answers
-      if (e == hipSuccess) RC_HIP(hipStreamSynchronize(s));
-      if (e == hipSuccess && *word == 0u) return rc::set_error(RAJA_CDNA4_ERROR_HIP, "no answer from the key sample");
-      if (e != hipSuccess && e != hipErrorNotReady) RC_HIP(e);
+      rc::TimedScope ts("radix_hist", s);
+      hipLaunchKernelGGL((hist_kernel<K>), dim3(hist_blocks(n)), dim3(256), 0, s, keys, n, descending != 0, mem.hist,
+                         mem.desc, mem.lsd_desc_words, &plan->sample_ok);
+      RC_HIP(hipGetLastError());
     }
-    if (a.levels == 2 && *word == 1u) return RAJA_CDNA4_SUCCESS;
+    uint32_t answer = 0;
+    RC_TRY(rc::wait_word(host + 1, s, &answer));
+    if (answer == 1u)
+    {
+      rc::TimedScope ts("radix_hist", s);
+      hipLaunchKernelGGL((digits_kernel<K>), dim3(1), dim3(256), 0, s, mem.hist, (uint32_t)n, mem.host + 2);
+      RC_HIP(hipGetLastError());
+      return rc::wait_word(host + 2, s, digits);
+    }
   }
   {
     rc::TimedScope ts("partition_hist", s);
@@ -610,9 +668,9 @@ int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* a
     {
       const int64_t want = rc::ceil_div(n, (int64_t)kHist1Keys);
       hipLaunchKernelGGL((hist1_kernel<K>), dim3((unsigned)(want < 512 ? want : 512)), dim3(256), 0, s, keys, n,
-                         flip, plan, count1, d0, a.ntiles * kRowStride);
+                         flip, plan, count1, d0, a.ntiles * kRowStride, mem.hist, mem.lsd_desc_words);
       hipLaunchKernelGGL((plan1_kernel<K>), dim3(1), dim3(256), 0, s, plan, count1, (uint32_t)n, most0, most1, window,
-                         (uint32_t)a.ngroups, start, host_ok);
+                         (uint32_t)a.ngroups, start, mem.hist, mem.host);
     }
     else
     {
@@ -629,11 +687,11 @@ int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* a
       hipLaunchKernelGGL((rows_kernel<K>), dim3(kRadix), dim3(1024), 0, s, plan, (const uint32_t*)alt_k, blocks,
                          rows, total, largest);
       hipLaunchKernelGGL((plan2_kernel<K>), dim3(1), dim3(256), 0, s, plan, total, largest, most0, most1,
-                         (uint32_t)a.tile, base, tile0, host_ok);
+                         (uint32_t)a.tile, base, tile0, mem.host);
     }
     RC_HIP(hipGetLastError());
   }
-  RC_HIP(hipEventRecord(ready, s));
+  RC_HIP(hipEventRecord(mem.ready, s));
   // The first scatter is launched before the decision is known here (it checks
   // it on the device), so the wait below passes while it runs.  The gate (one
   // lookback launch at a time on the device) is held for each scatter's
@@ -661,9 +719,13 @@ int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* a
     }
     RC_HIP(hipGetLastError());
   }
-  RC_HIP(hipEventSynchronize(ready));
-  const uint32_t ok = *(volatile uint32_t*)host_ok;
-  if (ok == 0u) return RAJA_CDNA4_SUCCESS;
+  RC_HIP(hipEventSynchronize(mem.ready));
+  const uint32_t ok = host[0];
+  if (ok == 0u)
+  {
+    *digits = host[2];
+    return RAJA_CDNA4_SUCCESS;
+  }
   if (a.levels == 2)
   {
     rc::LookbackGate gate(s);
@@ -684,21 +746,17 @@ int partition_typed(int dtype, int descending, K* keys, V* vals, int64_t n, K* a
 }
 
 template<typename K>
-int partition_key(int dtype, int val_bytes, int descending, void* keys, void* vals, int64_t n, void* ak,
-                  void* av, char* aux, uint32_t* desc, uint32_t* host_ok, hipEvent_t ready, hipStream_t s,
-                  bool* done)
+int partition_key(int dtype, int val_bytes, int descending, void* keys, void* vals, int64_t n,
+                  const rsort::PartitionMem& mem, hipStream_t s, bool* done, uint32_t* digits)
 {
   switch (val_bytes)
   {
     case 0:
-      return partition_typed<K, uint32_t, false>(dtype, descending, (K*)keys, nullptr, n, (K*)ak, nullptr, aux,
-                                                 desc, host_ok, ready, s, done);
+      return partition_typed<K, uint32_t, false>(dtype, descending, (K*)keys, nullptr, n, mem, s, done, digits);
     case 4:
-      return partition_typed<K, uint32_t, true>(dtype, descending, (K*)keys, (uint32_t*)vals, n, (K*)ak,
-                                                (uint32_t*)av, aux, desc, host_ok, ready, s, done);
+      return partition_typed<K, uint32_t, true>(dtype, descending, (K*)keys, (uint32_t*)vals, n, mem, s, done, digits);
     default:
-      return partition_typed<K, uint64_t, true>(dtype, descending, (K*)keys, (uint64_t*)vals, n, (K*)ak,
-                                                (uint64_t*)av, aux, desc, host_ok, ready, s, done);
+      return partition_typed<K, uint64_t, true>(dtype, descending, (K*)keys, (uint64_t*)vals, n, mem, s, done, digits);
   }
 }
 
@@ -715,10 +773,13 @@ int partition_levels(int kb, int vb, int64_t n)
   if (n <= kRadix * (int64_t)4700) return 1;
   if (n > kFine * (int64_t)4700) return 0;
   // Per sort, LSD against partition, uniform keys: u64 keys + 4-byte values 2^22
-  // 279 / 152 us, 2^26 3.07 / 1.46 ms; u32 keys + 4-byte values 2^23 189 / 203 us,
-  // 2^24 328 / 286, 2^26 1112 / 998, 2^28 4.07 / 3.50 ms, + 8-byte values 2^24
-  // 468 / 372 us; u32 keys alone 2^24 262 / 261 us, 2^27 1.44 / 1.63 ms.  A rejected
-  // span pays about 13 us, so 4-byte keys start at 2^25 (607 / 550 us).
+  // 279 / 162 us, 2^24 877 / 411 us; u32 keys + 4-byte values 2^23 186 / 192 us,
+  // 2^24 319 / 295, 2^25 608 / 559, 2^26 1111 / 1002, 2^28 4.07 / 3.50 ms, + 8-byte
+  // values 2^23 243 / 213, 2^24 467 / 381 us; u32 keys alone 2^24 262 / 261 us, 2^27
+  // 1.44 / 1.63 ms.  Refused spans pay 5 to 8 us: 3 to 4 % of a sort of few distinct
+  // 4-byte keys below 2^25 (2^24 150 / 154 us), 1 to 2.5 % there and less above.
+  // 4-byte keys start at 2^25: the gain at 2^24 (8 to 18 % of even keys) is left
+  // for the key sets that would pay for it.
   if (kb == 8) return n >= ((int64_t)1 << 22) ? 2 : 0;
   return (vb > 0 && n >= ((int64_t)1 << 25)) ? 2 : 0;
 }
@@ -728,14 +789,13 @@ size_t partition_aux_bytes(int kb, int vb, int64_t n) { return Aux(kb, vb, n).by
 int64_t partition_desc_rows(int kb, int vb, int64_t n) { return Aux(kb, vb, n).ntiles + kRadix; }
 
 int partition_sort(int key_dtype, int val_bytes, int descending, void* keys, void* vals, int64_t n,
-                   void* alt_keys, void* alt_vals, char* aux, uint32_t* desc, uint32_t* host_ok,
-                   hipEvent_t ready, hipStream_t s, bool* done)
+                   const PartitionMem& mem, hipStream_t s, bool* done, uint32_t* digits)
 {
   *done = false;
+  *digits = 0u;
 #define RSORT_PART(CODE, K)                                                                               \
   case CODE:                                                                                              \
-    return partition_key<K>(key_dtype, val_bytes, descending, keys, vals, n, alt_keys, alt_vals, aux, desc, \
-                            host_ok, ready, s, done);
+    return partition_key<K>(key_dtype, val_bytes, descending, keys, vals, n, mem, s, done, digits);
   switch (key_dtype)
   {
     RSORT_PART(RAJA_CDNA4_U32, uint32_t)

@@ -227,6 +227,24 @@ int ensure_tmp(StreamCtx* c, size_t bytes)
   return grow(c, &c->tmp, &c->tmp_cap, bytes, false);
 }
 
+int wait_word(const volatile uint32_t* word, hipStream_t s, uint32_t* out)
+{
+  for (uint32_t polls = 1; (*out = *word) == 0u; ++polls)
+  {
+    __builtin_ia32_pause();
+    // about every millisecond: a query can queue a marker behind the kernel
+    // that answers, which then holds up the next one
+    if ((polls & 0xFFFFu) != 0u) continue;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    RC_HIP(e);
+    RC_HIP(hipStreamSynchronize(s));
+    *out = *word;
+    return *out ? RAJA_CDNA4_SUCCESS : set_error(RAJA_CDNA4_ERROR_HIP, "no answer from the device");
+  }
+  return RAJA_CDNA4_SUCCESS;
+}
+
 bool timing_enabled() { return g_timing; }
 
 TimedScope::TimedScope(const char* n, hipStream_t s) : name(n), stream(s)

@@ -68,6 +68,11 @@ int ensure_tmp(StreamCtx* c, size_t bytes);
 
 int num_cus();
 
+// Waits until a kernel queued on `s` has stored something but 0 into a word of
+// pinned host memory, and gives it.  The host looks at the word, and now and
+// then at the stream: one that failed never answers.
+int wait_word(const volatile uint32_t* word, hipStream_t s, uint32_t* out);
+
 // Kernel timing (HIP events around launches on the launch stream).
 bool timing_enabled();
 struct TimedScope

@@ -8,8 +8,8 @@
 // Design (8-bit digits, P = 8*sizeof(key)/8 passes):
 //   1. one read of all keys builds the P digit histograms (LDS counters per
 //      block, wave-uniform digits added once per wave, then global atomics);
-//   2. the host reads the histograms back for large inputs and skips every
-//      pass whose digit is the same for all keys;
+//   2. for large inputs a small kernel tells the host which digits differ, and
+//      every pass whose digit is the same for all keys is skipped;
 //   3. each pass is one kernel: each block owns one tile (16384 keys of 32
 //      bits; 32 consecutive tiles of every 256 go to one XCD), loads its keys,
 //      ranks them inside each wave by 8 ballots (peer lanes
@@ -23,6 +23,7 @@
 //      launch or device counter is needed.
 // Ranking follows input order inside a wave (item j, then lane) and across
 // waves and tiles, so the sort is stable.
+#include "digit_hist.hpp"
 #include "local_sort.hpp"
 #include "ops.hpp"
 #include "onesweep.hpp"
@@ -34,148 +35,6 @@
 
 namespace
 {
-// ---- 1. all-pass digit histograms ------------------------------------------
-// Counts the N keys every lane of the wave holds (all of them valid) into
-// s_hist, bin b's copy c at word b * C + c, lane l counting into copy l % C.
-// A digit that is the same for all 64 * N keys is added once: the test is
-// an OR over the keys of (bits ^ lane 0's first bits), one ballot per digit.
-template<typename K, bool DESC, int P, int N, int C>
-__device__ __forceinline__ void count_full_wave(const K (&k)[N], uint32_t* s_hist, int lane)
-{
-  using bits_t = typename KeyTraits<K>::bits_t;
-  const bits_t b0 = KeyTraits<K>::to_bits(k[0]);
-  bits_t f = 0;
-  if constexpr (sizeof(bits_t) == 4)
-  {
-    f = (bits_t)__builtin_amdgcn_readfirstlane((int)b0);
-  }
-  else
-  {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b0);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b0 >> 32));
-    f = ((bits_t)hi << 32) | lo;
-  }
-  bits_t x = 0;
-#pragma unroll
-  for (int q = 0; q < N; ++q) x |= KeyTraits<K>::to_bits(k[q]) ^ f;
-#pragma unroll
-  for (int p = 0; p < P; ++p)
-  {
-    if (ballot(((x >> (8 * p)) & (bits_t)0xFF) != 0) == 0ull)
-    {
-      const uint32_t d0 = (uint32_t)((DESC ? ~f : f) >> (8 * p)) & (kRadix - 1);
-      if (lane == 0) atomicAdd(&s_hist[(p * kRadix + d0) * C], (uint32_t)(wave_size * N));
-    }
-    else
-    {
-      uint32_t* const h = s_hist + p * kRadix * C + (lane % C);
-#pragma unroll
-      for (int q = 0; q < N; ++q) atomicAdd(&h[digit_of<K, DESC>(k[q], 8 * p) * C], 1u);
-    }
-  }
-}
-
-// Each wave streams 64 lanes x U x 16-byte vectors per iteration (U vector
-// loads in flight per lane) and counts every digit of every key with LDS
-// atomics; a digit shared by all keys of a full iteration is added once
-// (constant high digits of small keys would otherwise serialise 64 lanes on
-// one LDS word).
-template<typename K, bool DESC, int P>
-__global__ __launch_bounds__(256) void hist_kernel(const K* __restrict__ keys, int64_t n,
-                                                   uint32_t* __restrict__ hist,
-                                                   uint32_t* __restrict__ desc0,
-                                                   int64_t desc0_words)
-{
-  constexpr int VEC = 16 / sizeof(K);
-  constexpr int U = 4;
-  constexpr int PER_WAVE = wave_size * U * VEC;
-  typedef K vec_t __attribute__((ext_vector_type(16 / sizeof(K))));
-  // kCopies counters per bin, side by side (bin b's copy c is word
-  // b * kCopies + c), lane l counting into copy l % kCopies: lanes of one
-  // atomic instruction that meet the same bin use different words in
-  // different banks.  2^28 keys: 0.283 ms with one copy, 0.239 ms with 4
-  // copies as separate histograms, 0.229 / 0.212 / 0.27 ms with 4 / 8 / 16
-  // side-by-side copies (copy l / 8 instead of l % 8: 0.285 ms).
-  constexpr int kCopies = 8;
-  __shared__ uint32_t s_hist[kCopies * P * kRadix];
-  for (int i = threadIdx.x; i < kCopies * P * kRadix; i += 256) s_hist[i] = 0u;
-  __syncthreads();
-  const int lane = lane_id();
-  const bool aligned = ((uintptr_t)keys % 16) == 0;
-  const int64_t nwaves = (int64_t)gridDim.x * (256 / wave_size);
-  for (int64_t base = ((int64_t)blockIdx.x * (256 / wave_size) + wave_id()) * PER_WAVE; base < n;
-       base += nwaves * PER_WAVE)
-  {
-    K k[U * VEC];
-    const bool full = aligned && base + PER_WAVE <= n;
-    if (full)
-    {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-      {
-        const vec_t x = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(keys + base + ((int64_t)u * wave_size + lane) * VEC));
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) k[u * VEC + e] = x[e];
-      }
-    }
-    else
-    {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-      {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e)
-        {
-          const int64_t i = base + ((int64_t)u * wave_size + lane) * VEC + e;
-          k[u * VEC + e] = (i < n) ? keys[i] : K(0);
-        }
-      }
-    }
-    if (full)
-    {
-      count_full_wave<K, DESC, P, U * VEC, kCopies>(k, s_hist, lane);
-      continue;
-    }
-#pragma unroll
-    for (int q = 0; q < U * VEC; ++q)
-    {
-      const int64_t i = base + ((int64_t)(q / VEC) * wave_size + lane) * VEC + (q % VEC);
-      const bool valid = full || i < n;
-      // valid lanes of one item form a prefix in lane order
-      const uint64_t vmask = ballot(valid);
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-      {
-        const uint32_t d = digit_of<K, DESC>(k[q], 8 * p);
-        const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
-        const bool uniform = (ballot(d == d0 || !valid) == ~0ull) && (vmask & 1ull);
-        if (uniform)
-        {
-          if (lane == 0) atomicAdd(&s_hist[(p * kRadix + d0) * kCopies], (uint32_t)__popcll(vmask));
-        }
-        else if (valid)
-        {
-          atomicAdd(&s_hist[(p * kRadix + d) * kCopies], 1u);
-        }
-      }
-    }
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < P * kRadix; i += 256)
-  {
-    uint32_t c = 0;
-#pragma unroll
-    for (int r = 0; r < kCopies; ++r) c += s_hist[i * kCopies + r];
-    if (c) atomic_add_agent(&hist[i], c);
-  }
-  // Clear the descriptors the first pass will use.
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < desc0_words; i += stride)
-  {
-    desc0[i] = 0u;
-  }
-}
-
 // Working memory of one sort: alternate key/value buffers, the digit
 // histograms and two descriptor arrays.
 template<typename K, typename V, bool HAS_VALS>
@@ -357,12 +216,13 @@ int seg_sort_core(const K* in_k, const V* in_v, K* out_k, V* out_v, K* alt_k, V*
 // Sort (in_keys, in_vals) into (keys, vals); in_keys == keys sorts in place.
 // tmp holds SortWs::tmp_bytes(), desc_mem SortWs::desc_bytes (its contents
 // are ignored: the histogram kernel clears the first array and every pass
-// clears the next).  With `pinned` (>= hist bytes of pinned host memory) the
-// histograms are read back -- one stream synchronisation -- to skip passes
-// whose digit is the same for every key.
+// clears the next).  With `pinned` (a word of pinned host memory) the host waits
+// for the word of active digits, to skip passes whose digit is the same for
+// every key.  `digits` not 0: that word, the histograms and the first pass's
+// descriptors being there already.
 template<typename K, typename V, bool HAS_VALS, bool DESC>
 int sort_core(const K* in_keys, const V* in_vals, K* keys, V* vals, int64_t n, hipStream_t s,
-              char* tmp, uint32_t* desc_mem, uint32_t* pinned, int items = 0)
+              char* tmp, uint32_t* desc_mem, uint32_t* pinned, int items = 0, uint32_t digits = 0)
 {
   using S = SortShape<K, V, HAS_VALS>;
   constexpr int P = (int)sizeof(K);
@@ -374,36 +234,23 @@ int sort_core(const K* in_keys, const V* in_vals, K* keys, V* vals, int64_t n, h
   uint32_t* desc[2] = {desc_mem, desc_mem + w.desc_words};
   const bool inplace = (const void*)in_keys == (const void*)keys;
 
+  if (digits == 0u)
   {
     rc::TimedScope ts("radix_hist", s);
     hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, hist, (int64_t)P * kRadix);
-    const int64_t want = rc::ceil_div(n, (int64_t)256 * 64);
-    const int64_t cap = (int64_t)rc::num_cus() * 16;
-    const unsigned grid = (unsigned)(want < 1 ? 1 : (want < cap ? want : cap));
-    hipLaunchKernelGGL((hist_kernel<K, DESC, P>), dim3(grid), dim3(256), 0, s, in_keys, n, hist,
-                       desc[0], w.desc_words);
+    hipLaunchKernelGGL((hist_kernel<K>), dim3(hist_blocks(n)), dim3(256), 0, s, in_keys, n, DESC, hist, desc[0],
+                       w.desc_words, (const uint32_t*)nullptr);
     RC_HIP(hipGetLastError());
-  }
-  bool active[P];
-  int npass = P;
-  for (int p = 0; p < P; ++p) active[p] = true;
-  if (pinned && n >= (int64_t)1 << 18)
-  {
-    RC_HIP(hipMemcpyAsync(pinned, hist, (size_t)P * kRadix * sizeof(uint32_t),
-                          hipMemcpyDeviceToHost, s));
-    RC_HIP(hipStreamSynchronize(s));
-    for (int p = 0; p < P; ++p)
+    digits = kDigitsKnown | ((1u << P) - 1u);
+    if (pinned && n >= (int64_t)1 << 18)
     {
-      for (int dd = 0; dd < kRadix; ++dd)
-      {
-        if ((int64_t)pinned[p * kRadix + dd] == n)
-        {
-          active[p] = false;
-          --npass;
-        }
-      }
+      *(volatile uint32_t*)pinned = 0u;
+      hipLaunchKernelGGL((digits_kernel<K>), dim3(1), dim3(256), 0, s, hist, (uint32_t)n, pinned);
+      RC_HIP(hipGetLastError());
+      RC_TRY(rc::wait_word(pinned, s, &digits));
     }
   }
+  const int npass = __builtin_popcount(digits & ~kDigitsKnown);
   rc::LookbackGate gate(s);  // one lookback launch at a time on the device
   RC_TRY(gate.status());
   // Out of place, an even pass count starts into the alternate buffers and
@@ -416,7 +263,7 @@ int sort_core(const K* in_keys, const V* in_vals, K* keys, V* vals, int64_t n, h
   int q = 0;
   for (int p = 0; p < P; ++p)
   {
-    if (!active[p]) continue;
+    if (((digits >> p) & 1u) == 0u) continue;
     K* kdst = to_alt ? alt_keys : keys;
     V* vdst = to_alt ? alt_vals : vals;
     rc::TimedScope ts("onesweep_pass", s);
@@ -497,6 +344,7 @@ int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
   constexpr int kb = (int)sizeof(K), vb = HAS_VALS ? (int)sizeof(V) : 0;
   const bool part = !lsd_only && pinned && rsort::partition_levels(kb, vb, n) > 0;
   size_t tmp = w.tmp_bytes(), desc = w.desc_bytes;
+  uint32_t digits = 0;
   if (part)
   {
     tmp += rsort::partition_aux_bytes(kb, vb, n);
@@ -508,13 +356,14 @@ int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
   {
     if (!c->ready) RC_HIP(hipEventCreateWithFlags(&c->ready, hipEventDisableTiming));
     char* const t = (char*)c->tmp;
+    const rsort::PartitionMem mem{t, t + w.keys_bytes, t + w.tmp_bytes(), (uint32_t*)c->sort_desc,
+                                  (uint32_t*)(t + w.keys_bytes + w.vals_bytes), w.desc_words, pinned, c->ready};
     bool done = false;
-    RC_TRY(rsort::partition_sort(rk::dtype_code<K>(), vb, DESC ? 1 : 0, keys, vals, n, t, t + w.keys_bytes,
-                                 t + w.tmp_bytes(), (uint32_t*)c->sort_desc, pinned, c->ready, s, &done));
+    RC_TRY(rsort::partition_sort(rk::dtype_code<K>(), vb, DESC ? 1 : 0, keys, vals, n, mem, s, &done, &digits));
     if (done) return RAJA_CDNA4_SUCCESS;
   }
   return sort_core<K, V, HAS_VALS, DESC>(keys, vals, keys, vals, n, s, (char*)c->tmp,
-                                         (uint32_t*)c->sort_desc, pinned, items);
+                                         (uint32_t*)c->sort_desc, pinned, items, digits);
 }
 
 template<typename K>

@@ -114,14 +114,25 @@ void failed_upload()
 }
 
 // ---- the lookback gate -------------------------------------------------------------
-// What the partition's kernels leave in pinned memory when it takes the keys
-// (arguments as in partition_sort.hip).
-void take_partition(const std::string& kernel, void** args)
+// What a sort's kernels leave in pinned memory (arguments as in
+// partition_sort.hip and digit_hist.hpp).
+constexpr uint32_t kTwoDigits = 0x80000005u;  // the keys differ in digits 0 and 2
+void answer(const std::string& kernel, void** args, bool sample, bool counts)
 {
-  if (kernel.find("sample_kernel") != std::string::npos) **(volatile uint32_t**)args[8] = 2u;
-  if (kernel.find("plan1_kernel") != std::string::npos) **(volatile uint32_t**)args[8] = 1u;
-  if (kernel.find("plan2_kernel") != std::string::npos) **(volatile uint32_t**)args[8] = 1u;
+  auto host = [&](int arg) { return *(volatile uint32_t**)args[arg]; };
+  auto is = [&](const char* name) { return kernel.find(name) != std::string::npos; };
+  if (is("sample_kernel")) *host(10) = sample ? 2u : 1u;
+  if (is("plan1_kernel"))
+  {
+    host(9)[0] = sample && counts ? 1u : 0u;
+    host(9)[2] = sample ? 0u : kTwoDigits;
+  }
+  if (is("plan2_kernel")) *host(8) = counts ? 1u : 0u;
+  if (is("digits_kernel")) *host(2) = kTwoDigits;
 }
+void take_partition(const std::string& k, void** a) { answer(k, a, true, true); }
+void sample_refuses(const std::string& k, void** a) { answer(k, a, false, false); }
+void counts_refuse(const std::string& k, void** a) { answer(k, a, true, false); }
 
 // While a sort waits on the host, a scan of many tiles on another thread and
 // stream must go through: the wait may be for work which that thread has yet
@@ -274,7 +285,7 @@ void tuner_shapes()
     CHECK(rec::count("launch", "sample_kernel") + rec::count("launch", "span_sort_kernel") == 0,
           "n = %lld: not the digit passes", (long long)n);
   }
-  rec::on_launch = nullptr;  // pinned memory stays 0: the partition refuses
+  rec::on_launch = sample_refuses;
   rec::clear();
   CHECK(tune(1, RAJA_CDNA4_I32, 1 << 20, nullptr) == 0, "tune");
   CHECK(shapes("scan_kernel") == (std::set<unsigned>{32, 64, 128}), "%zu scan tiles measured",
@@ -304,6 +315,51 @@ void tuner_shapes()
     CHECK(shapes("scan_kernel") == std::set<unsigned>{tuned ? 32u : 128u}, "scan tile");
   }
 }
+
+// ---- spans that the partition refuses -------------------------------------------------
+// A span that the sample refuses has its digits counted once, by the kernel
+// after the sample, and goes on with the digit passes: nothing is copied back
+// and the host waits once.  One that only the counts refuse starts over.
+void refused_spans()
+{
+  auto sort = ENTRY(raja_cdna4_sort_pairs);
+  const int64_t most = 1 << 22;
+  std::vector<uint64_t> keys((size_t)most);
+  std::vector<uint32_t> vals((size_t)most);
+  for (const auto& [dtype, n] : {std::pair<int, int64_t>{RAJA_CDNA4_U32, 1 << 20}, {RAJA_CDNA4_U64, 1 << 22}})
+  {
+    const bool one_level = n == 1 << 20;
+    for (int how = 0; how < 2; ++how)
+    {
+      rec::on_launch = how == 0 ? sample_refuses : counts_refuse;
+      for (int rep = 0; rep < 2; ++rep)  // the first call grows the scratch
+      {
+        rec::clear();
+        CHECK(sort(dtype, keys.data(), vals.data(), 4, n, 0, nullptr) == 0, "sort");
+      }
+      const size_t hists = rec::count("launch", "11hist_kernel");
+      const size_t scatters = rec::count("launch", "MapDigit");
+      const size_t passes = rec::count("launch", "onesweep_kernel") - scatters;
+      CHECK(passes == 2, "%zu passes for two digits", passes);
+      CHECK(rec::count("copy_async") == 0 && rec::count("stream_wait") == 0, "%zu copies, %zu waits",
+            rec::count("copy_async"), rec::count("stream_wait"));
+      CHECK(rec::count("launch", "local_groups") == 0, "block sorts");
+      if (how == 0)
+      {
+        CHECK(hists == (one_level ? 0 : 1), "%zu digit histograms after the sample", hists);
+        CHECK(rec::count("launch", "clear_words") == 0, "cleared again");
+        CHECK(scatters == (one_level ? 1 : 0), "%zu scatters", scatters);
+        CHECK(rec::count("launch", "hist1_kernel") == (one_level ? 1 : 0) && rec::count("launch", "hist2_kernel") == 0,
+              "counts");
+      }
+      else
+      {
+        CHECK(hists == (one_level ? 1 : 2), "%zu digit histograms after the counts", hists);
+      }
+    }
+  }
+  rec::on_launch = nullptr;
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -320,7 +376,8 @@ int main(int argc, char** argv)
                                                       {"gate_across_waits", gate_across_waits},
                                                       {"batched_sort_scratch", batched_sort_scratch},
                                                       {"noalloc_order", noalloc_order},
-                                                      {"tuner_shapes", tuner_shapes}};
+                                                      {"tuner_shapes", tuner_shapes},
+                                                      {"refused_spans", refused_spans}};
   const auto it = tests.find(argv[2]);
   if (it == tests.end()) return 2;
   it->second();

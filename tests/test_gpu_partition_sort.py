@@ -104,6 +104,16 @@ def test_counts_reject_what_the_sample_allows(raja, name, n):
     check(raja, name, 4, False, "spike", n)
 
 
+@pytest.mark.parametrize("name,n", [
+    ("u32", (1 << 18) + 1), ("i32", ONE), ("f32", ONE - 5), ("u64", (1 << 18) + 3), ("f64", ONE), ("i64", (1 << 22) + 1),
+    ("f64", (1 << 22) + 7), ("i32", (1 << 25) + 1)])
+def test_refused_keys(raja, name, n):
+    """Keys whose digits the partition counts after its sample has refused them:
+    in place at any alignment, both directions, 0, 4 and 8 value bytes."""
+    for vb, desc, shift in ((4, False, 1), (0, True, 0), (8, True, 3), (4, False, 0)):
+        check(raja, name, vb, desc, "few", n, shift)
+
+
 def test_sorted_and_reversed(raja):
     for n in (1_000_003, 5_000_011):
         for rev in (False, True):

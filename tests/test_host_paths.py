@@ -51,3 +51,9 @@ def test_tuner_measures_and_takes_the_shapes_it_names(exe, tmp_path):
     """Each candidate runs its own tile (digit passes for sorts, whatever the
     keys), and a recorded full tile is the full tile."""
     run(exe, "tuner_shapes", tmp_path)
+
+
+def test_refused_spans_count_their_digits_once(exe, tmp_path):
+    """A span that the partition's sample refuses goes from the sample to one
+    digit histogram and the passes, with no copy back to the host."""
+    run(exe, "refused_spans", tmp_path)
