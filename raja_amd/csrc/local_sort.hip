@@ -3,8 +3,9 @@
 //
 // The work is split by range length, each class with a block as large as its
 // longest range: one wave per range of up to 64 keys, 128 x 4 threads x keys
-// up to 512, 256 x 8 up to 2048, 640 x 8 up to 5120 and 1024 x 8 up to 8192.  A block holds its
-// keys and values in registers, reads and writes memory once and coalesced.
+// up to 512, 256 x 8 up to 2048, 640 x 8 up to 5120 and 1024 x 8 up to 8192
+// (small batches: the last for all).  A block holds its keys and values in
+// registers, reads and writes memory once and coalesced.
 //
 // Bounded by LDS work, not by memory, so the keys are placed with one LDS
 // atomic each instead of one wave ranking per 8-bit digit:
@@ -680,12 +681,22 @@ __global__ __launch_bounds__(1024) void lsd_kernel(const K* in_keys, const V* in
   }
 }
 
-// One span, placement or passes.
+// Placement or passes: one span (segs nullptr), or a record per block.
 template<typename K, typename V, bool HAS_VALS, int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) void span_sort_kernel(const K* in_keys, const V* in_vals, K* out_keys,
-                                                          V* out_vals, int n, bits_of<K> flip)
+                                                          V* out_vals, const rs::SortSeg* __restrict__ segs, int n,
+                                                          bits_of<K> flip)
 {
   __shared__ LocalLds<K, V, HAS_VALS, BLOCK, ITEMS> s;
+  if (segs)
+  {
+    const rs::SortSeg sg = segs[blockIdx.x];
+    in_keys += uniform(sg.in_keys);
+    in_vals += uniform(sg.in_vals);
+    out_keys += uniform(sg.out_keys);
+    out_vals += uniform(sg.out_vals);
+    n = (int)uniform(sg.n);
+  }
   const int per = items_of<BLOCK>(n);
   const int wbase = __builtin_amdgcn_readfirstlane(wave_id()) * wave_size * per;
   if (local_sort_bins<K, V, HAS_VALS, BLOCK, ITEMS>(s, in_keys, in_vals, out_keys, out_vals, n, per, wbase, flip))
@@ -697,6 +708,15 @@ __global__ __launch_bounds__(BLOCK) void span_sort_kernel(const K* in_keys, cons
 }
 
 constexpr int64_t kLsdBlocks = 512;
+
+// Batches of up to this many ranges, whatever their lengths, are one launch of
+// span_sort_kernel's 1024-thread block (two per CU): by classes they are up to
+// six launches in a row, each of which leaves most of the chip idle.
+// By classes / in one launch, u32 keys and 4-byte values, lengths 2^10 to 2^13:
+// 64 ranges 41.8 / 17.0 us, 512 46.6 / 26.1, 1024 50.3 / 41.6, 2048 69 / 74;
+// 2^4 to 2^9: 64 16.2 / 9.0, 512 18.0 / 13.9, 768 18.4 / 18.9, 1024 18.6 / 23.9;
+// u64 keys and 8-byte values 2^4 to 2^9: 512 19.0 / 18.0.
+constexpr int64_t kOneLaunch = 512;
 
 template<typename K, typename V, bool HAS_VALS>
 int launch_groups(int descending, const void* ik, const void* iv, void* ok_, void* ov, const uint32_t* start,
@@ -731,11 +751,21 @@ int launch_classes(const K* ik, const V* iv, K* ok, V* ov, bits_of<K> flip, cons
   {
     const int n = (int)span;
     if (n > rsort::kLocalMax[2])  // 1024 threads: the one block has the chip to itself
-      hipLaunchKernelGGL((span_sort_kernel<K, V, HAS_VALS, 1024, 8>), dim3(1), dim3(1024), 0, s, ik, iv, ok, ov, n, flip);
+      hipLaunchKernelGGL((span_sort_kernel<K, V, HAS_VALS, 1024, 8>), dim3(1), dim3(1024), 0, s, ik, iv,
+                         ok, ov, d_segs, n, flip);
     else if (n > rsort::kLocalMax[1])
-      hipLaunchKernelGGL((span_sort_kernel<K, V, HAS_VALS, 256, 8>), dim3(1), dim3(256), 0, s, ik, iv, ok, ov, n, flip);
+      hipLaunchKernelGGL((span_sort_kernel<K, V, HAS_VALS, 256, 8>), dim3(1), dim3(256), 0, s, ik, iv,
+                         ok, ov, d_segs, n, flip);
     else
-      hipLaunchKernelGGL((span_sort_kernel<K, V, HAS_VALS, 128, 4>), dim3(1), dim3(128), 0, s, ik, iv, ok, ov, n, flip);
+      hipLaunchKernelGGL((span_sort_kernel<K, V, HAS_VALS, 128, 4>), dim3(1), dim3(128), 0, s, ik, iv,
+                         ok, ov, d_segs, n, flip);
+    RC_HIP(hipGetLastError());
+    return RAJA_CDNA4_SUCCESS;
+  }
+  if (first[rsort::kLocalClasses] <= kOneLaunch)
+  {
+    hipLaunchKernelGGL((span_sort_kernel<K, V, HAS_VALS, 1024, 8>), dim3((unsigned)first[rsort::kLocalClasses]),
+                       dim3(1024), 0, s, ik, iv, ok, ov, d_segs, 0, flip);
     RC_HIP(hipGetLastError());
     return RAJA_CDNA4_SUCCESS;
   }

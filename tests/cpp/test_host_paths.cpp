@@ -257,6 +257,28 @@ void noalloc_order()
   }
 }
 
+// A small batch is one launch, whatever its segments' lengths; a large one a
+// launch per length class and one for what those leave to the passes.
+void batched_sort_launches()
+{
+  auto create = ENTRY(raja_cdna4_segments_create);
+  auto destroy = ENTRY(raja_cdna4_segments_destroy);
+  auto sort = ENTRY(raja_cdna4_segmented_sort_pairs);
+  for (int count : {1, 60, 512, 513})
+  {
+    std::vector<int64_t> off = {0};
+    for (int g = 0; g < count; ++g) off.push_back(off.back() + 2 + 1297 * g % 8190);
+    std::vector<uint32_t> keys((size_t)off.back()), vals(keys.size());
+    raja_cdna4_segments_s* p = nullptr;
+    CHECK(create(off.data(), count, &p) == 0, "create");
+    rec::clear();
+    CHECK(sort(p, RAJA_CDNA4_U32, keys.data(), vals.data(), 4, 0, nullptr) == 0, "sort");
+    const size_t want = count <= 512 ? 1 : 6;
+    CHECK(rec::count("launch") == want, "%d segments: %zu launches", count, rec::count("launch"));
+    CHECK(destroy(p) == 0, "destroy");
+  }
+}
+
 // ---- shape tuning --------------------------------------------------------------------
 // The tuner's candidates run the kernels that they name, and a recorded full
 // tile is taken, not the tile that untuned spans of that length take.
@@ -377,7 +399,8 @@ int main(int argc, char** argv)
                                                       {"batched_sort_scratch", batched_sort_scratch},
                                                       {"noalloc_order", noalloc_order},
                                                       {"tuner_shapes", tuner_shapes},
-                                                      {"refused_spans", refused_spans}};
+                                                      {"refused_spans", refused_spans},
+                                                      {"batched_sort_launches", batched_sort_launches}};
   const auto it = tests.find(argv[2]);
   if (it == tests.end()) return 2;
   it->second();

@@ -88,12 +88,13 @@ def test_span_and_segment_sorts_of_short_ranges(raja, name, vb):
             assert same_bits(host(k, p), p[o]), (how, desc, len(p))
             if vb:
                 assert np.array_equal(w.cpu().numpy(), v[o]), (how, desc, len(p))
-        # as segments
-        off = np.concatenate([[0], np.cumsum([len(p) for p in parts])])
-        plan = raja.Segments(off)
-        k, w = dev(np.concatenate(parts)), (dev(np.concatenate(vals)) if vb else None)
-        raja.segmented_sort_pairs(plan, k, w, comp)
-        assert same_bits(host(k, parts[0]), np.concatenate([p[o] for p, o in zip(parts, want)])), how
-        if vb:
-            assert np.array_equal(w.cpu().numpy(), np.concatenate([v[o] for v, o in zip(vals, want)])), how
-        plan.close()
+        # as segments: few (one launch for all) and over 512 (a launch per length class)
+        for reps in (1, 24):
+            off = np.concatenate([[0], np.cumsum([len(p) for p in parts] * reps)])
+            plan = raja.Segments(off)
+            k, w = dev(np.concatenate(parts * reps)), (dev(np.concatenate(vals * reps)) if vb else None)
+            raja.segmented_sort_pairs(plan, k, w, comp)
+            assert same_bits(host(k, parts[0]), np.concatenate([p[o] for p, o in zip(parts, want)] * reps)), (how, reps)
+            if vb:
+                assert np.array_equal(w.cpu().numpy(), np.concatenate([v[o] for v, o in zip(vals, want)] * reps)), (how, reps)
+            plan.close()

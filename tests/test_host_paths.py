@@ -57,3 +57,7 @@ def test_refused_spans_count_their_digits_once(exe, tmp_path):
     """A span that the partition's sample refuses goes from the sample to one
     digit histogram and the passes, with no copy back to the host."""
     run(exe, "refused_spans", tmp_path)
+
+
+def test_small_batch_of_short_sorts_is_one_launch(exe, tmp_path):
+    run(exe, "batched_sort_launches", tmp_path)
