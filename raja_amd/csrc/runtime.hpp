@@ -13,6 +13,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "RAJA/policy/cdna4/intrinsics.hpp"
 #include "raja_cdna4.h"
 
@@ -53,7 +55,8 @@ struct StreamCtx
   void* tmp = nullptr;           // general temporaries (alt buffers, partials)
   size_t tmp_cap = 0;
   void* pinned = nullptr;        // 64 KiB pinned host staging
-  void* small = nullptr;         // 64 KiB device slots of fixed place: marks and results of one call
+  void* small = nullptr;         // 64 KiB device slots of fixed place: marks of one call
+  std::mutex small_lock;         // held while a call that uses them is queued
   hipEvent_t ready = nullptr;    // recorded where a sort's host decision is known
   uint32_t scan_epoch = 0;       // tag of the latest scan's lookback descriptors
 };

@@ -337,7 +337,10 @@ int seg_sort(raja_cdna4_segments_s* p, K* keys, V* vals, int key_dtype, int val_
   {
     // The block sorts' marks, a byte per segment: in the stream's fixed slots
     // while they fit (no growth, so a capture needs no call of the same size
-    // before it, and a graph keeps a pointer that never moves).
+    // before it, and a graph keeps a pointer that never moves).  The lock
+    // keeps another thread's batch on this stream from coming between the
+    // kernel that writes them and the one that reads them.
+    std::lock_guard<std::mutex> g(c->small_lock);
     const size_t marks = (size_t)tab->first[rsort::kLocalClasses];
     uint8_t* redo = (uint8_t*)c->small;
     if (marks > rc::small_slot_bytes)

@@ -279,6 +279,43 @@ void batched_sort_launches()
   }
 }
 
+// Two threads' batches of short segments on one stream: the launches of one come
+// in a row, so neither reads marks that the other has written over.
+void batched_sorts_of_two_threads()
+{
+  auto create = ENTRY(raja_cdna4_segments_create);
+  auto sort = ENTRY(raja_cdna4_segmented_sort_pairs);
+  std::vector<int64_t> off = {0};
+  for (int g = 0; g < 3000; ++g) off.push_back(off.back() + 2 + 37 * g % 8190);
+  std::vector<uint32_t> keys((size_t)off.back()), vals(keys.size());
+  raja_cdna4_segments_s* p = nullptr;
+  CHECK(create(off.data(), (int64_t)off.size() - 1, &p) == 0, "create");
+  auto one = [&](int descending) {
+    return sort(p, RAJA_CDNA4_U32, keys.data(), vals.data(), 4, descending, nullptr);
+  };
+  CHECK(one(0) == 0, "sort");
+  std::vector<std::thread::id> order;
+  std::mutex m;
+  std::thread other;
+  rec::on_launch = [&](const std::string&, void**) {
+    bool first = false;
+    {
+      std::lock_guard<std::mutex> g(m);
+      first = order.empty();
+      order.push_back(std::this_thread::get_id());
+    }
+    if (!first) return;
+    other = std::thread([&] { CHECK(one(0) == 0, "sort"); });
+    std::this_thread::sleep_for(std::chrono::milliseconds(300));
+  };
+  CHECK(one(0) == 0, "sort");
+  other.join();
+  rec::on_launch = nullptr;
+  size_t turns = 0;
+  for (size_t i = 1; i < order.size(); ++i) turns += order[i] != order[i - 1];
+  CHECK(order.size() == 12 && turns == 1, "%zu launches, %zu changes of thread", order.size(), turns);
+}
+
 // ---- shape tuning --------------------------------------------------------------------
 // The tuner's candidates run the kernels that they name, and a recorded full
 // tile is taken, not the tile that untuned spans of that length take.
@@ -400,7 +437,8 @@ int main(int argc, char** argv)
                                                       {"noalloc_order", noalloc_order},
                                                       {"tuner_shapes", tuner_shapes},
                                                       {"refused_spans", refused_spans},
-                                                      {"batched_sort_launches", batched_sort_launches}};
+                                                      {"batched_sort_launches", batched_sort_launches},
+                                                      {"batched_sorts_of_two_threads", batched_sorts_of_two_threads}};
   const auto it = tests.find(argv[2]);
   if (it == tests.end()) return 2;
   it->second();

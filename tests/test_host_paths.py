@@ -61,3 +61,7 @@ def test_refused_spans_count_their_digits_once(exe, tmp_path):
 
 def test_small_batch_of_short_sorts_is_one_launch(exe, tmp_path):
     run(exe, "batched_sort_launches", tmp_path)
+
+
+def test_batched_sorts_of_two_threads_on_one_stream(exe, tmp_path):
+    run(exe, "batched_sorts_of_two_threads", tmp_path)
