@@ -53,9 +53,10 @@ def keys_of(name, how, n, g):
         raw[1:: n // 40] = torch.iinfo(INT[size]).min
     elif how == "normal":
         raw = (torch.randn(n, generator=g, device=DEV, dtype=torch.float64) * 2 ** 27).to(INT[size])
-    elif how == "spike":  # one bucket too full, too thin for the sample to see
+    elif how == "spike":  # one bucket too full, too thin for the sample to see: one level has
+        # buckets of up to 4700 on average and room for 5120, two levels far smaller ones
         raw = torch.randint(-2 ** 31, 2 ** 31, (n,), generator=g, device=DEV, dtype=INT[size])
-        raw[n // 2: n // 2 + 9000] = 12345
+        raw[n // 2: n // 2 + (1200 if n <= ONE else 9000)] = 12345
     else:
         raw = torch.randint(-2 ** 31, 2 ** 31, (n,), generator=g, device=DEV, dtype=torch.int64)
         if size == 8:
@@ -64,7 +65,20 @@ def keys_of(name, how, n, g):
     return raw, raw.view(U[name]) if name in U else raw
 
 
+def routed(raja, sort):
+    """Launches of the sort's phases: sample, counts, scatters, block sorts, digit passes."""
+    raja.timing_enable(True)
+    try:
+        raja.timing_reset()
+        sort()
+        return tuple(raja.timing_query(p)["count"] for p in (
+            "partition_sample", "partition_hist", "partition_scatter", "partition_local", "onesweep_pass"))
+    finally:
+        raja.timing_enable(False)
+
+
 def check(raja, name, vb, desc, how, n, shift=0):
+    """Sorts and compares; returns the sort's route."""
     g = torch.Generator(device=DEV)
     g.manual_seed(n + vb)
     raw, keys = keys_of(name, how, n, g)
@@ -75,11 +89,26 @@ def check(raja, name, vb, desc, how, n, shift=0):
     k = room[shift:]
     k.view(INT[size]).copy_(raw) if shift == 0 else room.view(INT[size])[shift:].copy_(raw)
     v = torch.arange(n, device=DEV, dtype=INT[vb]) if vb else None
-    raja.sort_pairs(k, v, raja.operators.greater if desc else raja.operators.less)
+    route = routed(raja, lambda: raja.sort_pairs(k, v, raja.operators.greater if desc else raja.operators.less))
     assert torch.equal(room.view(INT[size])[shift:], raw[order]), (name, vb, desc, how, n)
     if vb:
         assert torch.equal(v.to(torch.int64), order), (name, vb, desc, how, n)
     raja.device_status()
+    return route
+
+
+def levels(name, vb, n):
+    """Levels the partition has for a span of this length (0: digit passes)."""
+    if n < 1 << 18 or n > 65536 * 4700:
+        return 0
+    if n <= ONE:
+        return 1
+    if name[1:] == "64":
+        return 2 if n >= 1 << 22 else 0
+    return 2 if vb and n >= 1 << 25 else 0
+
+
+ACCEPTED = {0: (0, 0, 0, 0), 1: (1, 1, 1, 1), 2: (1, 1, 2, 1)}
 
 
 @pytest.mark.parametrize("name", ["u32", "i32", "f32", "u64", "i64", "f64"])
@@ -95,13 +124,17 @@ def test_key_sets(raja, name, how):
     ("i64", 8, ONE - 1), ("u32", 4, (1 << 25) + 7), ("u32", 8, (1 << 25) - 1), ("u32", 4, 9 * (1 << 24) + 11), ("u64", 0, 1 << 22),
     ("u64", 4, (1 << 24) + 3), ("i64", 8, 330 * 65536), ("i64", 0, 1200 * 65536), ("f64", 4, (1 << 23) + 1)])
 def test_lengths(raja, name, vb, n):
-    check(raja, name, vb, False, "uniform", n)
-    check(raja, name, vb, True, "uniform", n, shift=1)
+    want = ACCEPTED[levels(name, vb, n)]
+    assert check(raja, name, vb, False, "uniform", n)[:4] == want
+    assert check(raja, name, vb, True, "uniform", n, shift=1)[:4] == want
 
 
-@pytest.mark.parametrize("name,n", [("i32", 1 << 20), ("i32", (1 << 25) + 3), ("i64", 1 << 20), ("i64", 1 << 22)])
+@pytest.mark.parametrize("name,n", [("i32", ONE), ("i32", (1 << 25) + 3), ("i64", ONE), ("i64", 1 << 22)])
 def test_counts_reject_what_the_sample_allows(raja, name, n):
-    check(raja, name, 4, False, "spike", n)
+    """The sample and the counts run, the first scatter is launched and ends at
+    once, no block sorts follow: the digit passes sort."""
+    route = check(raja, name, 4, False, "spike", n)
+    assert route[:4] == (1, 1, 1, 0) and route[4] > 0
 
 
 @pytest.mark.parametrize("name,n", [
@@ -111,7 +144,10 @@ def test_refused_keys(raja, name, n):
     """Keys whose digits the partition counts after its sample has refused them:
     in place at any alignment, both directions, 0, 4 and 8 value bytes."""
     for vb, desc, shift in ((4, False, 1), (0, True, 0), (8, True, 3), (4, False, 0)):
-        check(raja, name, vb, desc, "few", n, shift)
+        route = check(raja, name, vb, desc, "few", n, shift)
+        # one level counts and launches its scatter without the answer, two levels do not
+        assert route[:4] == {0: (0, 0, 0, 0), 1: (1, 1, 1, 0), 2: (1, 0, 0, 0)}[levels(name, vb, n)]
+        assert route[4] > 0
 
 
 def test_sorted_and_reversed(raja):

@@ -341,8 +341,9 @@ def test_sort_pairs_skips_constant_digits(raja, orc, bits):
     """From 2^18 keys the digit passes whose digit is the same for every key
     are skipped: equal keys run none, 8-bit keys one and 24-bit keys three
     (an odd count, which in place ends with a copy back into the keys);
-    every result is the stable sort."""
-    for n in ((1 << 18) + 5, (1 << 20) + 3):
+    every result is the stable sort.  The passes are counted at lengths that
+    always take them; at the two others even keys are partitioned."""
+    for n in ((1 << 18) + 5, (1 << 20) + 3, 1_300_003, (1 << 21) + 17):
         print("sort skipping constant digits: n %d, %d-bit keys" % (n, bits), flush=True)
         k = torch.empty(n, dtype=torch.uint32, device=DEV)
         if bits == 0:
@@ -351,7 +352,15 @@ def test_sort_pairs_skips_constant_digits(raja, orc, bits):
             raja.fill(raja.FILL_U32_BITS, k, seed=5, a=bits)
         v = torch.arange(n, dtype=torch.int32, device=DEV)
         hk = to_np(k)
-        raja.sort_pairs(k, v)
+        raja.timing_enable(True)
+        try:
+            raja.timing_reset()
+            raja.sort_pairs(k, v)
+            passes = raja.timing_query("onesweep_pass")["count"]
+        finally:
+            raja.timing_enable(False)
+        if n > 256 * 4700:
+            assert passes == bits // 8, (n, bits)
         ek, ev = orc.seq_stable_sort_pairs(hk, np.arange(n, dtype=np.int32))
         assert np.array_equal(to_np(k), ek), (n, bits)
         assert np.array_equal(to_np(v), ev), (n, bits)
