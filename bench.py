@@ -4,11 +4,11 @@ Headline workload: radix sort_pairs of N = 2^28 uint32 keys uniform over
 [0, 2^32) with int32 iota values (the sort configuration of the reference
 study).  One step = one sort_pairs call on resident inputs; the pristine keys
 and values are restored by a device copy before each step, outside the
-per-step event pair.  value counts 68 bytes per pair whichever way the sort
-runs: the four LSD passes of 8-bit digits (read+write key and value, 16 each)
+per-step event pair.  value is a normalised rate: 68 bytes per pair whichever way the sort
+runs, the four LSD passes of 8-bit digits (read+write key and value, 16 each)
 and the histogram read (4).  moves_executed and moved_bytes_per_elem say what
 this run moved: 16 per executed move (an LSD pass, or a scatter or the block
-sorts of the partition) + 4 for the histogram read.
+sorts of the partition) + 4 for the histogram read.  hbm_frac is of those bytes.
 
 Also measured (reported under "ops"): the fused ReduceSum/Min/Max/MinLoc of
 N(0,1) FP64, exclusive_scan of int32 in [0,16), inclusive_scan of int64 and
@@ -143,10 +143,11 @@ def main():
     moved_per_elem = 16 * p_exec + 4
     ms = statistics.mean(step_ms)
     gbs = n * bytes_per_elem / (ms * 1e-3) / 1e9
+    moved_gbs = n * moved_per_elem / (ms * 1e-3) / 1e9
     pass_ms = passes["total_ms"] / max(1, passes["count"])
     pass_gbs = n * 16 / (pass_ms * 1e-3) / 1e9
-    log("bench: sort_pairs %.3f ms/step (%.1f GB/s, %d moves), onesweep pass %.3f ms (%.1f GB/s)"
-        % (ms, gbs, p_exec, pass_ms, pass_gbs))
+    log("bench: sort_pairs %.3f ms/step (%.1f GB/s at 68 B a pair; %d moves, %.1f GB/s moved), "
+        "onesweep scatter %.3f ms (%.1f GB/s)" % (ms, gbs, p_exec, moved_gbs, pass_ms, pass_gbs))
 
     # correctness of the last step (size-independent, exact)
     hk0 = keys0.view(torch.int32).cpu().numpy().view(np.uint32)
@@ -214,8 +215,8 @@ def main():
             "workload": "sort_pairs: N=2^%d uint32 keys uniform [0,2^32), int32 iota values, "
                         "ascending, stable (two onesweep scatters and block sorts, or LSD onesweep 8-bit digits)" % args.log2n,
             "n": n, "moves_executed": p_exec, "bytes_per_elem": bytes_per_elem,
-            "moved_bytes_per_elem": moved_per_elem, "moved_GB/s": round(n * moved_per_elem / (ms * 1e-3) / 1e9, 2),
-            "hbm_frac": round(gbs / PEAK_GBS, 4), "keys_per_s": round(n / (ms * 1e-3), 1),
+            "moved_bytes_per_elem": moved_per_elem, "moved_GB/s": round(moved_gbs, 2),
+            "hbm_frac": round(moved_gbs / PEAK_GBS, 4), "keys_per_s": round(n / (ms * 1e-3), 1),
             "result_exact": ok, "wall_s_timed_loop": round(wall, 3),
         },
         "roofline": {

@@ -225,7 +225,7 @@ __device__ __forceinline__ void write_sorted(LocalLds<K, V, HAS_VALS, BLOCK, ITE
 }
 
 // Bin placement; false (in every thread) if the bins are too uneven, before
-// anything is written.  *lo_out: the smallest ordered key.
+// anything is written.
 template<typename K, typename V, bool HAS_VALS, int BLOCK, int ITEMS>
 __device__ __forceinline__ bool local_sort_bins(LocalLds<K, V, HAS_VALS, BLOCK, ITEMS>& s, const K* in_keys,
                                                 const V* in_vals, K* out_keys, V* out_vals, int n, int per,
@@ -244,9 +244,9 @@ __device__ __forceinline__ bool local_sort_bins(LocalLds<K, V, HAS_VALS, BLOCK, 
   if constexpr (HAS_VALS) load_items(in_vals, n, per, wbase, lane, v);
   // Counter words per thread (two bins each): twice as many bins as keys where
   // the counters have room for them, else as many.
-  constexpr int MAXW = ITEMS >= 16 ? 8 : (ITEMS >= 8 ? 4 : 2);
+  constexpr int MAXW = ITEMS >= 8 ? 4 : 2;
   static_assert(MAXW * BLOCK <= L::CAP / 2, "counters fit their LDS");
-  const int words = per >= MAXW ? MAXW : (per > 4 ? 8 : (per > 2 ? 4 : (per > 1 ? 2 : 1)));
+  const int words = per >= MAXW ? MAXW : (per > 2 ? 4 : (per > 1 ? 2 : 1));
   const uint32_t nb = (uint32_t)(words * 2 * BLOCK);
   for (int q = 0; q < words; ++q) s.bin.cnt[q * BLOCK + tid] = 0u;
 
@@ -287,143 +287,143 @@ __device__ __forceinline__ bool local_sort_bins(LocalLds<K, V, HAS_VALS, BLOCK, 
   if (!narrow && !bin_of.ok) return false;
 
   uint32_t pos[ITEMS];
-    // bin << 16 | slot inside the bin
-    auto take_slot = [&](int j, uint32_t bin) {
-      const uint32_t sh = (bin & 1u) * 16u;
-      const uint32_t c = atomicAdd(&s.bin.cnt[bin >> 1], 1u << sh);
-      pos[j] = (bin << 16) | ((c >> sh) & 0xFFFFu);
-    };
-    if (narrow)
+  // bin << 16 | slot inside the bin
+  auto take_slot = [&](int j, uint32_t bin) {
+    const uint32_t sh = (bin & 1u) * 16u;
+    const uint32_t c = atomicAdd(&s.bin.cnt[bin >> 1], 1u << sh);
+    pos[j] = (bin << 16) | ((c >> sh) & 0xFFFFu);
+  };
+  if (narrow)
+  {
+    each([&](int j) {
+      again(k[j]);
+      take_slot(j, (uint32_t)((float)(uint32_t)(ordered<K>(k[j], flip) - lo) * inv));
+    });
+  }
+  else
+  {
+    each([&](int j) {
+      again(k[j]);
+      take_slot(j, bin_of(k[j], ordered<K>(k[j], flip)));
+    });
+  }
+  __syncthreads();
+  // Places of the bins: a thread's words in a row, one wave scan of the
+  // threads' sums, then the wave totals.
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  uint32_t w[MAXW], ex = 0;
+  u16x2 worst2 = {0, 0};
+  auto read_words = [&](auto count_c) {
+    constexpr int W = decltype(count_c)::value;
+    uint32_t sum = 0;
+#pragma unroll
+    for (int q = 0; q < W; ++q) w[q] = s.bin.cnt[tid * W + q];
+#pragma unroll
+    for (int q = 0; q < W; ++q)
     {
-      each([&](int j) {
-        again(k[j]);
-        take_slot(j, (uint32_t)((float)(uint32_t)(ordered<K>(k[j], flip) - lo) * inv));
-      });
+      sum += (w[q] & 0xFFFFu) + (w[q] >> 16);
+      worst2 = __builtin_elementwise_max(worst2, __builtin_bit_cast(u16x2, w[q]));
     }
+    uint32_t total;
+    (void)wave_scan(sum, rk::OpPlus<uint32_t>{}, 0u, ex, total);
+    if (lane == 0) s.scan[wave] = total;
+  };
+  auto write_words = [&](auto count_c) {
+    constexpr int W = decltype(count_c)::value;
+    uint32_t before = (lane & 15) < wave ? s.scan[lane & 15] : 0u;
+    before = __builtin_amdgcn_readfirstlane(row_sum(before));
+    uint32_t p = before + ex;
+#pragma unroll
+    for (int q = 0; q < W; ++q)
+    {
+      const uint32_t p1 = p + (w[q] & 0xFFFFu);
+      s.bin.cnt[tid * W + q] = p | (p1 << 16);
+      p = p1 + (w[q] >> 16);
+    }
+  };
+  auto by_words = [&](auto&& f) {
+    if (words == 1)
+      f(std::integral_constant<int, 1>{});
+    else if (words == 2)
+      f(std::integral_constant<int, 2>{});
+    else if (MAXW >= 4 && words == 4)
+      f(std::integral_constant<int, MAXW >= 4 ? 4 : 2>{});
     else
-    {
-      each([&](int j) {
-        again(k[j]);
-        take_slot(j, bin_of(k[j], ordered<K>(k[j], flip)));
+      f(std::integral_constant<int, MAXW>{});
+  };
+  by_words(read_words);
+  const uint32_t worst = worst2[0] > worst2[1] ? worst2[0] : worst2[1];
+  if (__syncthreads_or(worst > kMaxBin) != 0) return false;
+  by_words(write_words);
+  if (tid == 0) s.bin.cnt[nb / 2] = (uint32_t)n;
+  __syncthreads();
+  const uint16_t* const place = reinterpret_cast<const uint16_t*>(s.bin.cnt);
+  uint32_t share = 0;  // bit j: item j shares its bin
+  uint32_t* const s_comp = reinterpret_cast<uint32_t*>(s.buf);
+  auto put = [&](int j, auto&& store) {
+    const uint32_t bin = pos[j] >> 16;
+    const uint32_t first = place[bin], end = place[bin + 1];
+    store(first + (pos[j] & 0xFFFFu));
+    pos[j] = (end << 16) | first;
+    share |= (end - first > 1u) ? 1u << j : 0u;
+  };
+  auto comp_of = [&](int j) {
+    again(k[j]);
+    return ((uint32_t)(ordered<K>(k[j], flip) - lo) << ibits) | (uint32_t)(wbase + j * wave_size + lane);
+  };
+  if (narrow)
+  {
+    each([&](int j) { put(j, [&](uint32_t at) { s_comp[at] = comp_of(j); }); });
+  }
+  else
+  {
+    each([&](int j) {
+      put(j, [&](uint32_t at) {
+        s_keys[at] = k[j];
+        s.bin.idx[at] = (uint16_t)(wbase + j * wave_size + lane);
       });
+    });
+  }
+  __syncthreads();
+  if (narrow)
+  {
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+    {
+      if (j < per && ((share >> j) & 1u))
+      {
+        const uint32_t first = pos[j] & 0xFFFFu, end = pos[j] >> 16;
+        const uint32_t me = comp_of(j);
+        uint32_t r = first;
+        for (uint32_t q = first; q < end; ++q) r += s_comp[q] < me ? 1u : 0u;
+        pos[j] = r;
+      }
     }
-    __syncthreads();
-    // Places of the bins: a thread's words in a row, one wave scan of the
-    // threads' sums, then the wave totals.
-    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-    uint32_t w[MAXW], ex = 0;
-    u16x2 worst2 = {0, 0};
-    auto read_words = [&](auto count_c) {
-      constexpr int W = decltype(count_c)::value;
-      uint32_t sum = 0;
+  }
+  else
+  {
 #pragma unroll
-      for (int q = 0; q < W; ++q) w[q] = s.bin.cnt[tid * W + q];
-#pragma unroll
-      for (int q = 0; q < W; ++q)
+    for (int j = 0; j < ITEMS; ++j)
+    {
+      if (j < per && ((share >> j) & 1u))
       {
-        sum += (w[q] & 0xFFFFu) + (w[q] >> 16);
-        worst2 = __builtin_elementwise_max(worst2, __builtin_bit_cast(u16x2, w[q]));
-      }
-      uint32_t total;
-      (void)wave_scan(sum, rk::OpPlus<uint32_t>{}, 0u, ex, total);
-      if (lane == 0) s.scan[wave] = total;
-    };
-    auto write_words = [&](auto count_c) {
-      constexpr int W = decltype(count_c)::value;
-      uint32_t before = (lane & 15) < wave ? s.scan[lane & 15] : 0u;
-      before = __builtin_amdgcn_readfirstlane(row_sum(before));
-      uint32_t p = before + ex;
-#pragma unroll
-      for (int q = 0; q < W; ++q)
-      {
-        const uint32_t p1 = p + (w[q] & 0xFFFFu);
-        s.bin.cnt[tid * W + q] = p | (p1 << 16);
-        p = p1 + (w[q] >> 16);
-      }
-    };
-    auto by_words = [&](auto&& f) {
-      if (words == 1)
-        f(std::integral_constant<int, 1>{});
-      else if (words == 2)
-        f(std::integral_constant<int, 2>{});
-      else if (MAXW >= 4 && words == 4)
-        f(std::integral_constant<int, MAXW >= 4 ? 4 : 2>{});
-      else
-        f(std::integral_constant<int, MAXW>{});
-    };
-    by_words(read_words);
-    const uint32_t worst = worst2[0] > worst2[1] ? worst2[0] : worst2[1];
-    if (__syncthreads_or(worst > kMaxBin) != 0) return false;
-      by_words(write_words);
-      if (tid == 0) s.bin.cnt[nb / 2] = (uint32_t)n;
-      __syncthreads();
-      const uint16_t* const place = reinterpret_cast<const uint16_t*>(s.bin.cnt);
-      uint32_t share = 0;  // bit j: item j shares its bin
-      uint32_t* const s_comp = reinterpret_cast<uint32_t*>(s.buf);
-      auto put = [&](int j, auto&& store) {
-        const uint32_t bin = pos[j] >> 16;
-        const uint32_t first = place[bin], end = place[bin + 1];
-        store(first + (pos[j] & 0xFFFFu));
-        pos[j] = (end << 16) | first;
-        share |= (end - first > 1u) ? 1u << j : 0u;
-      };
-      auto comp_of = [&](int j) {
+        const uint32_t first = pos[j] & 0xFFFFu, end = pos[j] >> 16;
+        const uint32_t me = (uint32_t)(wbase + j * wave_size + lane);
         again(k[j]);
-        return ((uint32_t)(ordered<K>(k[j], flip) - lo) << ibits) | (uint32_t)(wbase + j * wave_size + lane);
-      };
-      if (narrow)
-      {
-        each([&](int j) { put(j, [&](uint32_t at) { s_comp[at] = comp_of(j); }); });
-      }
-      else
-      {
-        each([&](int j) {
-          put(j, [&](uint32_t at) {
-            s_keys[at] = k[j];
-            s.bin.idx[at] = (uint16_t)(wbase + j * wave_size + lane);
-          });
-        });
-      }
-      __syncthreads();
-      if (narrow)
-      {
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j)
+        const bits_t b = ordered<K>(k[j], flip);
+        uint32_t r = first;
+        for (uint32_t q = first; q < end; ++q)
         {
-          if (j < per && ((share >> j) & 1u))
-          {
-            const uint32_t first = pos[j] & 0xFFFFu, end = pos[j] >> 16;
-            const uint32_t me = comp_of(j);
-            uint32_t r = first;
-            for (uint32_t q = first; q < end; ++q) r += s_comp[q] < me ? 1u : 0u;
-            pos[j] = r;
-          }
+          const bits_t bq = ordered<K>(s_keys[q], flip);
+          r += (bq < b || (bq == b && s.bin.idx[q] < me)) ? 1u : 0u;
         }
+        pos[j] = r;
       }
-      else
-      {
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j)
-        {
-          if (j < per && ((share >> j) & 1u))
-          {
-            const uint32_t first = pos[j] & 0xFFFFu, end = pos[j] >> 16;
-            const uint32_t me = (uint32_t)(wbase + j * wave_size + lane);
-            again(k[j]);
-            const bits_t b = ordered<K>(k[j], flip);
-            uint32_t r = first;
-            for (uint32_t q = first; q < end; ++q)
-            {
-              const bits_t bq = ordered<K>(s_keys[q], flip);
-              r += (bq < b || (bq == b && s.bin.idx[q] < me)) ? 1u : 0u;
-            }
-            pos[j] = r;
-          }
-        }
-      }
-      __syncthreads();
-      write_sorted<K, V, HAS_VALS, BLOCK, ITEMS>(s, k, v, pos, out_keys, out_vals, n, per, wbase);
-      return true;
+    }
+  }
+  __syncthreads();
+  write_sorted<K, V, HAS_VALS, BLOCK, ITEMS>(s, k, v, pos, out_keys, out_vals, n, per, wbase);
+  return true;
 }
 
 // LSD passes of 8-bit digits over the digits that differ.
@@ -445,134 +445,134 @@ __device__ __forceinline__ void local_sort_lsd(LocalLds<K, V, HAS_VALS, BLOCK, I
   uint32_t pos[ITEMS];
   load_items(in_keys, n, per, wbase, lane, k);
   if constexpr (HAS_VALS) load_items(in_vals, n, per, wbase, lane, v);
-    const bits_t some = ordered<K>(in_keys[0], flip);
-    bits_t diff = 0;
+  const bits_t some = ordered<K>(in_keys[0], flip);
+  bits_t diff = 0;
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-    {
-      if (j < per && wbase + j * wave_size + lane < n) diff |= ordered<K>(k[j], flip) ^ some;
-    }
-    diff = wave_reduce(diff, rk::OpBitOr<bits_t>{});
-    __syncthreads();  // s.hi is read above
-    if (lane == 0) s.hi[wave] = diff;
-    __syncthreads();
+  for (int j = 0; j < ITEMS; ++j)
+  {
+    if (j < per && wbase + j * wave_size + lane < n) diff |= ordered<K>(k[j], flip) ^ some;
+  }
+  diff = wave_reduce(diff, rk::OpBitOr<bits_t>{});
+  __syncthreads();  // s.hi is read above
+  if (lane == 0) s.hi[wave] = diff;
+  __syncthreads();
 #pragma unroll
-    for (int w = 0; w < NW; ++w) diff |= s.hi[w];
-    // The last pass leaves the places in pos; before it, keys and values are
-    // moved through LDS.  No digit that differs: input order.
+  for (int w = 0; w < NW; ++w) diff |= s.hi[w];
+  // The last pass leaves the places in pos; before it, keys and values are
+  // moved through LDS.  No digit that differs: input order.
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) pos[j] = (uint32_t)(wbase + j * wave_size + lane);
-    bool first_pass = true;
+  for (int j = 0; j < ITEMS; ++j) pos[j] = (uint32_t)(wbase + j * wave_size + lane);
+  bool first_pass = true;
 #pragma unroll 1
-    for (int p = 0; p < P; ++p)
+  for (int p = 0; p < P; ++p)
+  {
+    if (((uint32_t)(diff >> (8 * p)) & 0xFFu) == 0u) continue;
+    if (!first_pass)
     {
-      if (((uint32_t)(diff >> (8 * p)) & 0xFFu) == 0u) continue;
-      if (!first_pass)
+      // to the places of the previous pass and back in input order of this one
+#pragma unroll
+      for (int j = 0; j < ITEMS; ++j)
       {
-        // to the places of the previous pass and back in input order of this one
+        if (j < per && wbase + j * wave_size + lane < n) s_keys[pos[j]] = k[j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < ITEMS; ++j)
+      {
+        const int i = wbase + j * wave_size + lane;
+        if (j < per && i < n) k[j] = s_keys[i];
+      }
+      __syncthreads();
+      if (HAS_VALS)
+      {
+        V* const s_vals = reinterpret_cast<V*>(s.buf);
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j)
         {
-          if (j < per && wbase + j * wave_size + lane < n) s_keys[pos[j]] = k[j];
+          if (j < per && wbase + j * wave_size + lane < n) s_vals[pos[j]] = v[j];
         }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j)
         {
           const int i = wbase + j * wave_size + lane;
-          if (j < per && i < n) k[j] = s_keys[i];
+          if (j < per && i < n) v[j] = s_vals[i];
         }
         __syncthreads();
-        if (HAS_VALS)
-        {
-          V* const s_vals = reinterpret_cast<V*>(s.buf);
-#pragma unroll
-          for (int j = 0; j < ITEMS; ++j)
-          {
-            if (j < per && wbase + j * wave_size + lane < n) s_vals[pos[j]] = v[j];
-          }
-          __syncthreads();
-#pragma unroll
-          for (int j = 0; j < ITEMS; ++j)
-          {
-            const int i = wbase + j * wave_size + lane;
-            if (j < per && i < n) v[j] = s_vals[i];
-          }
-          __syncthreads();
-        }
       }
-      first_pass = false;
-      for (int i = tid; i < NW * kRadix; i += BLOCK) s.lsd.whist[i] = 0u;
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j)
-      {
-        if (j < per)
-        {
-          const bool valid = wbase + j * wave_size + lane < n;
-          again(k[j]);
-          const uint32_t d = (uint32_t)(ordered<K>(k[j], flip) >> (8 * p)) & (kRadix - 1);
-          // peers as in onesweep_kernel: one extract and two v_bitop3 per bit
-          const uint64_t vb = ballot(valid);
-          uint32_t pl = (uint32_t)vb, ph = (uint32_t)(vb >> 32);
-#pragma unroll
-          for (int b = 0; b < 8; ++b)
-          {
-            int32_t sx = __builtin_amdgcn_sbfe((int32_t)d, b, 1);
-            asm volatile("" : "+v"(sx));
-            const uint64_t bal = ballot(sx != 0);
-            pl = __builtin_amdgcn_bitop3_b32(pl, (uint32_t)bal, (uint32_t)sx, 0x90);
-            ph = __builtin_amdgcn_bitop3_b32(ph, (uint32_t)(bal >> 32), (uint32_t)sx, 0x90);
-          }
-          const uint32_t lower = __builtin_amdgcn_mbcnt_hi(ph, __builtin_amdgcn_mbcnt_lo(pl, 0u));
-          uint32_t c = 0;
-          if (valid) c = s.lsd.whist[wave * kRadix + d];
-          pos[j] = c + lower;
-          asm volatile("" : "+v"(pos[j]));
-          if (valid && lower == 0)
-          {
-            s.lsd.whist[wave * kRadix + d] = c + (uint32_t)__builtin_popcount(pl) + (uint32_t)__builtin_popcount(ph);
-          }
-          __builtin_amdgcn_sched_barrier(0);  // one item at a time: few live masks
-        }
-      }
-      __syncthreads();
-      for (int d0 = 0; d0 < kRadix; d0 += BLOCK)
-      {
-        const int d = d0 + tid;
-        uint32_t ex = 0, total = 0;
-        if (d < kRadix)
-        {
-#pragma unroll
-          for (int w = 0; w < NW; ++w)
-          {
-            const uint32_t c = s.lsd.whist[w * kRadix + d];
-            s.lsd.whist[w * kRadix + d] = total;
-            total += c;
-          }
-          uint32_t sum;
-          (void)wave_scan(total, rk::OpPlus<uint32_t>{}, 0u, ex, sum);
-          s.lsd.tstart[d] = ex;
-          if (lane == 0) s.scan[d / wave_size] = sum;
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j)
-      {
-        if (j < per && wbase + j * wave_size + lane < n)
-        {
-          again(k[j]);
-          const uint32_t d = (uint32_t)(ordered<K>(k[j], flip) >> (8 * p)) & (kRadix - 1);
-          uint32_t base = s.lsd.tstart[d] + s.lsd.whist[wave * kRadix + d];
-#pragma unroll
-          for (int x = 0; x < kRadix / wave_size - 1; ++x) base += (x < (int)(d / wave_size)) ? s.scan[x] : 0u;
-          pos[j] += base;
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      __syncthreads();
     }
+    first_pass = false;
+    for (int i = tid; i < NW * kRadix; i += BLOCK) s.lsd.whist[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+    {
+      if (j < per)
+      {
+        const bool valid = wbase + j * wave_size + lane < n;
+        again(k[j]);
+        const uint32_t d = (uint32_t)(ordered<K>(k[j], flip) >> (8 * p)) & (kRadix - 1);
+        // peers as in onesweep_kernel: one extract and two v_bitop3 per bit
+        const uint64_t vb = ballot(valid);
+        uint32_t pl = (uint32_t)vb, ph = (uint32_t)(vb >> 32);
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+        {
+          int32_t sx = __builtin_amdgcn_sbfe((int32_t)d, b, 1);
+          asm volatile("" : "+v"(sx));
+          const uint64_t bal = ballot(sx != 0);
+          pl = __builtin_amdgcn_bitop3_b32(pl, (uint32_t)bal, (uint32_t)sx, 0x90);
+          ph = __builtin_amdgcn_bitop3_b32(ph, (uint32_t)(bal >> 32), (uint32_t)sx, 0x90);
+        }
+        const uint32_t lower = __builtin_amdgcn_mbcnt_hi(ph, __builtin_amdgcn_mbcnt_lo(pl, 0u));
+        uint32_t c = 0;
+        if (valid) c = s.lsd.whist[wave * kRadix + d];
+        pos[j] = c + lower;
+        asm volatile("" : "+v"(pos[j]));
+        if (valid && lower == 0)
+        {
+          s.lsd.whist[wave * kRadix + d] = c + (uint32_t)__builtin_popcount(pl) + (uint32_t)__builtin_popcount(ph);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one item at a time: few live masks
+      }
+    }
+    __syncthreads();
+    for (int d0 = 0; d0 < kRadix; d0 += BLOCK)
+    {
+      const int d = d0 + tid;
+      uint32_t ex = 0, total = 0;
+      if (d < kRadix)
+      {
+#pragma unroll
+        for (int w = 0; w < NW; ++w)
+        {
+          const uint32_t c = s.lsd.whist[w * kRadix + d];
+          s.lsd.whist[w * kRadix + d] = total;
+          total += c;
+        }
+        uint32_t sum;
+        (void)wave_scan(total, rk::OpPlus<uint32_t>{}, 0u, ex, sum);
+        s.lsd.tstart[d] = ex;
+        if (lane == 0) s.scan[d / wave_size] = sum;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+    {
+      if (j < per && wbase + j * wave_size + lane < n)
+      {
+        again(k[j]);
+        const uint32_t d = (uint32_t)(ordered<K>(k[j], flip) >> (8 * p)) & (kRadix - 1);
+        uint32_t base = s.lsd.tstart[d] + s.lsd.whist[wave * kRadix + d];
+#pragma unroll
+        for (int x = 0; x < kRadix / wave_size - 1; ++x) base += (x < (int)(d / wave_size)) ? s.scan[x] : 0u;
+        pos[j] += base;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+  }
   write_sorted<K, V, HAS_VALS, BLOCK, ITEMS>(s, k, v, pos, out_keys, out_vals, n, per, wbase);
 }
 
