@@ -220,7 +220,7 @@ def main():
             "result_exact": ok, "wall_s_timed_loop": round(wall, 3),
         },
         "roofline": {
-            "bound": "hbm", "kernel": "onesweep_pass",
+            "bound": "hbm", "kernel": "onesweep_kernel (scatter or digit pass)",
             "achieved": round(pass_gbs, 2), "peak": PEAK_GBS, "unit": "GB/s",
             "frac": round(pass_gbs / PEAK_GBS, 4),
             "algorithmic_bytes_per_launch": n * 16,
@@ -257,15 +257,15 @@ def tune_shapes(R, torch, n, measure=True):
                 log("bench: shape tuning of %s: %s" % (name, e))
             choice, tuned = R.tune_query(op, dt, n)
         out[name] = {"choice": choice, "tuned": tuned, "measured_now": measured}
-        log("bench: shape %s at n=%d: %s (0 = default)" % (name, n, choice))
+        log("bench: shape %s at n=%d: %s (0 = the full tile)" % (name, n, choice))
     return out
 
 
-TRAFFIC_FILE = os.path.join("profiles", "onesweep_pass_sort_pairs_2p28_hbm_traffic.md")
+TRAFFIC_FILE = os.path.join("profiles", "sort_pairs_2p28_hbm_traffic.md")
 
 
 def committed_traffic(log2n):
-    """HBM bytes per onesweep pass at N=2^28, from the committed FETCH_SIZE /
+    """HBM bytes per onesweep scatter of the partition at N=2^28 (mean of the two), from the committed FETCH_SIZE /
     WRITE_SIZE summary (counter runs scaled by a plain copy of known size)."""
     if log2n != 28:
         return None, None

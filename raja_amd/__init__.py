@@ -611,8 +611,8 @@ def autotune(op, dtype, n):
 
 
 def tune_query(op, dtype, n):
-    """(choice, tuned): the shape a call of (op, dtype, n) takes; choice 0 is
-    the default shape."""
+    """(choice, tuned): the tuned shape of (op, dtype, n); choice 0 is the full
+    tile.  Untuned lengths take the library's own rule."""
     _prep()
     c, t = ctypes.c_int(), ctypes.c_int()
     _check(lib().raja_cdna4_tune_query(op, _DTYPES[dtype], int(n), ctypes.byref(c), ctypes.byref(t)))

@@ -30,7 +30,7 @@
 // 47 us, 2^20 127 / 63, 2^25 607 / 550, 2^28 4.07 / 3.50 ms (counts 0.20, scatters 1.00
 // and 1.05, local sorts 1.27 ms); u64 keys and 4-byte values 2^20 203 / 71 us, 2^26
 // 3.08 / 1.46 ms.  The scatters run at the onesweep pass's rate; the local sorts
-// are bound by vector instructions (about 160 per 64 keys).
+// are bound by vector instructions (138 per 64 pairs).
 #include "partition_sort.hpp"
 
 #include "digit_hist.hpp"

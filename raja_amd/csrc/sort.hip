@@ -336,7 +336,7 @@ int sort_impl(K* keys, V* vals, int64_t n, hipStream_t s, int items = -1)
   rc::StreamCtx* c = nullptr;
   RC_TRY(rc::get_ctx(s, &c));
   const SortWs<K, V, HAS_VALS> w(n, items);
-  // Under stream capture the histogram readback (a host wait) cannot run:
+  // Under stream capture the word of active digits (a host wait) cannot be had:
   // every pass is executed instead, with the same result.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   RC_HIP(hipStreamIsCapturing(s, &cap));

@@ -2,7 +2,7 @@
 graph and replayed: every replay, with eager work and synchronisations
 between replays, gives the bits of the eager calls.  Captured scans clear
 their lookback descriptors with a kernel node (no memset node); a captured
-sort runs every digit pass (no host readback of the histograms)."""
+sort runs every digit pass (the host does not ask which digits differ)."""
 import numpy as np
 import pytest
 import torch
