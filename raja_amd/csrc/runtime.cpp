@@ -236,7 +236,11 @@ int wait_word(const volatile uint32_t* word, hipStream_t s, uint32_t* out)
     // that answers, which then holds up the next one
     if ((polls & 0xFFFFu) != 0u) continue;
     const hipError_t e = hipStreamQuery(s);
-    if (e == hipErrorNotReady) continue;
+    if (e == hipErrorNotReady)
+    {
+      (void)hipGetLastError();  // an answer, not an error that a later launch check should find
+      continue;
+    }
     RC_HIP(e);
     RC_HIP(hipStreamSynchronize(s));
     *out = *word;

@@ -35,6 +35,7 @@ inline std::map<const void*, std::string> g_kernels;
 inline std::map<void*, size_t> g_live;  // device blocks
 inline int g_fail_malloc = 0, g_fail_copy = 0;  // > 0: the n-th one from now fails
 inline bool g_capturing = false;
+inline int g_not_ready = 0;  // > 0: so many stream queries answer "not ready", as an error that stays
 inline hipError_t g_last = hipSuccess;
 // Called at a launch (stands in for what the kernel would leave in pinned
 // memory) and at a host wait, outside the lock.
@@ -252,7 +253,7 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st)
 hipError_t hipStreamQuery(hipStream_t)
 {
   rec::waited("stream_query");
-  return hipSuccess;
+  return rec::g_not_ready > 0 && rec::g_not_ready-- > 0 ? rec::fail(hipErrorNotReady) : hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s)
 {

@@ -316,6 +316,48 @@ void batched_sorts_of_two_threads()
   CHECK(order.size() == 12 && turns == 1, "%zu launches, %zu changes of thread", order.size(), turns);
 }
 
+// ---- a stream with a long queue --------------------------------------------------------
+// The answers of a sort's kernels come late: the queries in between are no
+// errors, the calls after them succeed, and a stream that ends without an answer
+// is reported.
+void late_answers()
+{
+  auto sort = ENTRY(raja_cdna4_sort_pairs);
+  const int64_t n = 1 << 22;
+  std::vector<uint64_t> keys((size_t)n);
+  std::vector<uint32_t> vals((size_t)n);
+  std::vector<std::function<void()>> late;
+  bool never = false;
+  rec::on_launch = [&](const std::string& kernel, void** args) {
+    volatile uint32_t* w = nullptr;
+    if (kernel.find("sample_kernel") != std::string::npos) w = *(volatile uint32_t**)args[10];
+    if (kernel.find("digits_kernel") != std::string::npos) w = *(volatile uint32_t**)args[2];
+    const uint32_t v = kernel.find("sample_kernel") != std::string::npos ? 1u : kTwoDigits;
+    if (w && !never)
+    {
+      rec::g_not_ready = 3;
+      late.push_back([w, v] { *w = v; });
+    }
+  };
+  rec::on_wait = [&](const char*) {
+    if (rec::g_not_ready == 1 && !late.empty())
+    {
+      late.back()();
+      late.pop_back();
+    }
+  };
+  for (const auto& [dtype, len] : {std::pair<int, int64_t>{RAJA_CDNA4_U64, n}, {RAJA_CDNA4_U32, 2000000}})
+  {
+    rec::clear();
+    CHECK(sort(dtype, keys.data(), vals.data(), 4, len, 0, nullptr) == 0, "sort with late answers");
+    CHECK(rec::count("launch", "onesweep_kernel") == 2, "%zu passes", rec::count("launch", "onesweep_kernel"));
+  }
+  never = true;
+  CHECK(sort(RAJA_CDNA4_U64, keys.data(), vals.data(), 4, n, 0, nullptr) != 0, "a missing answer goes unreported");
+  rec::on_launch = nullptr;
+  rec::on_wait = nullptr;
+}
+
 // ---- shape tuning --------------------------------------------------------------------
 // The tuner's candidates run the kernels that they name, and a recorded full
 // tile is taken, not the tile that untuned spans of that length take.
@@ -437,6 +479,7 @@ int main(int argc, char** argv)
                                                       {"noalloc_order", noalloc_order},
                                                       {"tuner_shapes", tuner_shapes},
                                                       {"refused_spans", refused_spans},
+                                                      {"late_answers", late_answers},
                                                       {"batched_sort_launches", batched_sort_launches},
                                                       {"batched_sorts_of_two_threads", batched_sorts_of_two_threads}};
   const auto it = tests.find(argv[2]);

@@ -158,3 +158,20 @@ def test_sorted_and_reversed(raja):
             k, v = raw.clone(), torch.arange(n, device=DEV, dtype=torch.int32)
             raja.sort_pairs(k, v)
             assert torch.equal(k, x) and torch.equal(v, raw), (n, rev)
+
+
+@pytest.mark.parametrize("name,how,n", [("u64", "uniform", 1 << 22), ("u64", "few", 1 << 22), ("u32", "uniform", 2_000_003)])
+def test_behind_a_long_queue(raja, name, how, n):
+    """The host polls the device's answers while tens of milliseconds of other
+    work on the stream come first."""
+    room = torch.empty(1 << 28, dtype=torch.int32, device=DEV)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(n)
+    raw, keys = keys_of(name, how, n, g)
+    order = torch.sort(bits_of(raw, name), stable=True).indices
+    k, v = keys.clone(), torch.arange(n, device=DEV, dtype=torch.int32)
+    torch.cuda.synchronize()
+    for i in range(60):
+        room.fill_(i)
+    raja.sort_pairs(k, v)
+    assert torch.equal(k.view(raw.dtype), raw[order]) and torch.equal(v.to(torch.int64), order)

@@ -65,3 +65,9 @@ def test_small_batch_of_short_sorts_is_one_launch(exe, tmp_path):
 
 def test_batched_sorts_of_two_threads_on_one_stream(exe, tmp_path):
     run(exe, "batched_sorts_of_two_threads", tmp_path)
+
+
+def test_answers_that_come_late(exe, tmp_path):
+    """A sort behind a long queue polls its answers and asks the stream now and
+    then: "not ready" is no error, a missing answer is."""
+    run(exe, "late_answers", tmp_path)
